@@ -46,6 +46,40 @@ def test_products_of_tiny_values(on_hip, scale):
     assert (np.abs(got - A64 @ B64) <= 192 * 2.0 ** -23 * (np.abs(A64) @ np.abs(B64))).all()
 
 
+# Root mean square of the error over sum |a b|.  Normal operands: rounding of a running sum of j terms is at most 2^-24 of its
+# size, sqrt(j); eight roundings per 16 k (the fp32 instructions) make 2^-24 / sqrt(3) * k / 2 over 2 / pi * k = 2.7e-8 at any
+# length, six (the three terms) 2.3e-8.  A row's figure, from 160 or 192 elements, stays within twice that.
+ROUNDING = 2.0 * 2.7e-8
+
+
+def _rounding(got, A, B, axis=None):
+    A64, B64 = A.astype(np.float64), B.astype(np.float64)
+    return np.sqrt((((got.astype(np.float64) - A64 @ B64) / (np.abs(A64) @ np.abs(B64))) ** 2).mean(axis))
+
+
+@pytest.mark.parametrize("k", [100, 192, 4096])
+@pytest.mark.parametrize("sa,sb", [(1e-35, 1e20), (1e-37, 1e30), (1e-38, 1e30), (1e-40, 1e36), (1e-41, 1e37), (1e30, 1e-38), (1e36, 1e-40)])
+def test_operands_below_the_range_of_three_terms(on_hip, sa, sb, k):
+    """Small operands against large ones: the sums are of ordinary size, the third term of the small operand is not."""
+    rng = np.random.RandomState(11)
+    A, B = (sa * rng.standard_normal((192, k))).astype(np.float32), (sb * rng.standard_normal((k, 160))).astype(np.float32)
+    assert (_rounding(_sgemm(on_hip, 0, 0, A, B), A, B, 1) <= ROUNDING).all()
+
+
+@pytest.mark.parametrize("k", [100, 192, 4096])
+@pytest.mark.parametrize("scale", [1e-34, 1e-36, 1e-38, 1e-40, 1e-42])
+def test_small_rows_and_columns_beside_ordinary_ones(on_hip, scale, k):
+    rng = np.random.RandomState(12)
+    A, B = rng.standard_normal((192, k)), 1e10 * rng.standard_normal((k, 160))
+    A[5] *= scale
+    A[70] *= scale
+    A, B = A.astype(np.float32), B.astype(np.float32)
+    assert (_rounding(_sgemm(on_hip, 0, 0, A, B), A, B, 1) <= ROUNDING).all()
+    assert (_rounding(_sgemm(on_hip, 0, 1, A, B), A, B, 1) <= ROUNDING).all()
+    At, Bt = np.ascontiguousarray(B.T), np.ascontiguousarray(A.T)
+    assert (_rounding(_sgemm(on_hip, 1, 0, At, Bt), At, Bt, 0) <= ROUNDING).all()
+
+
 @pytest.mark.parametrize("k", [64, 250, 4096])
 def test_products_with_infinities_and_nan_are_those_of_fp32(on_hip, k):
     rng = np.random.RandomState(9)
