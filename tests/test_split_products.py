@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from lantern_amd import Tensor, TensorR, _lib, gradR_loss
+from tests.util import Dev
 
 pytestmark = pytest.mark.gpu
 
@@ -124,3 +125,39 @@ def test_convolutions_with_infinities(on_hip, geom):
         ok = np.isfinite(want)
         # sums of `terms` products of size about one: that many roundings of a unit of a running sum below 8 sqrt(terms)
         assert (np.abs(got - want)[ok] <= terms * 2.0 ** -23 * 8 * np.sqrt(terms)).all()
+
+
+@pytest.mark.parametrize("dims", [(8, 64, 28, 28, 128, 3, 3, 1, 1, 1, 1), (4, 256, 14, 14, 256, 1, 1, 1, 1, 0, 0), (6, 96, 15, 15, 160, 3, 3, 1, 1, 1, 1),
+                                  (16, 32, 28, 28, 32, 3, 3, 1, 1, 1, 1), (8, 128, 28, 28, 256, 1, 1, 2, 2, 0, 0)], ids=lambda d: "x".join(map(str, d)))
+@pytest.mark.parametrize("plant", ["infinity", "small"])
+def test_plain_tile_plans_give_the_same_bits_around_what_the_terms_cannot_hold(on_hip, dims, plant, monkeypatch):
+    """Deterministic mode leaves the choice among the plans with whole tiles to a timing, so an infinity or a value below the range
+    of the three terms may change the arithmetic of the 32x32 blocks it is in only, which all tile shapes share."""
+    dev = Dev(on_hip)
+    lib = on_hip.lib
+    N, Cc, H, W, K, R, S, sH, sW, pH, pW = dims
+    P, Q = (H + 2 * pH - R) // sH + 1, (W + 2 * pW - S) // sW + 1
+    rng = np.random.RandomState(13)
+    x, w, dy = rng.randn(N, Cc, H, W).astype(np.float32), (rng.randn(K, Cc, R, S) / np.sqrt(Cc * R * S)).astype(np.float32), rng.randn(N, K, P, Q).astype(np.float32)
+    value = np.float32(np.inf) if plant == "infinity" else np.float32(1.2345678e-38)
+    x[1, 3, 4, 6] = dy[1, 3, 4, 5] = dy[N - 1, K - 1, P - 1, 0] = x[N - 1, 2, H - 4, 0] = value       # (even rows and columns: under a stride of two too)
+    if plant == "small":
+        w[7, 1, 0, 0] = w[K - 1, Cc - 1, R - 1, S - 1] = value
+    xd, wd, dyd = dev.up(x), dev.up(w), dev.up(dy)
+    ny, nx = N * K * P * Q, N * Cc * H * W
+    lib.lh_set_deterministic(1)
+    try:
+        outs = {}
+        for plan in (3, 2, 1, 10):
+            monkeypatch.setenv("LH_FORCE_PLAN", str(plan))
+            y = dev.up(np.full(ny, 7.0, np.float32)); lib.lh_conv2d_fwd(xd.ptr, wd.ptr, 0, y.ptr, *dims)
+            dx = dev.up(np.full(nx, 7.0, np.float32)); lib.lh_conv2d_bwd_data(dyd.ptr, wd.ptr, dx.ptr, 0.0, *dims)
+            dev.check()
+            outs[plan] = (dev.down(y, (ny,)).copy(), dev.down(dx, (nx,)).copy())
+        for plan in (2, 1, 10):
+            np.testing.assert_array_equal(outs[plan][0], outs[3][0], err_msg="forward, plan %d against plan 3" % plan)
+            np.testing.assert_array_equal(outs[plan][1], outs[3][1], err_msg="input gradient, plan %d against plan 3" % plan)
+        assert plant == "small" or (np.isinf(outs[3][0]).any() and np.isinf(outs[3][1]).any())
+    finally:
+        monkeypatch.delenv("LH_FORCE_PLAN", raising=False)
+        lib.lh_set_deterministic(0)
