@@ -58,6 +58,24 @@ def _rounding(got, A, B, axis=None):
     return np.sqrt((((got.astype(np.float64) - A64 @ B64) / (np.abs(A64) @ np.abs(B64))) ** 2).mean(axis))
 
 
+@pytest.mark.parametrize("tt", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 8])
+@pytest.mark.parametrize("spread", [0.0, 2.0])
+def test_short_sums_are_no_further_off_than_fused_multiply_adds(on_hip, tt, k, spread):
+    """One product is the rounded product itself; over a few the error is at most that of a chain of fused multiply-adds (here: of
+    float64 sums rounded after every term; 2 % for the sampling over half a million sums)."""
+    rng = np.random.RandomState(14)
+    draw = lambda *s: (rng.standard_normal(s) * np.exp(spread * rng.standard_normal(s))).astype(np.float32)      # noqa: E731
+    A, B = draw(512, k), draw(k, 1024)
+    got = _sgemm(on_hip, tt[0], tt[1], A, B)
+    chain = np.zeros((512, 1024), np.float32)
+    for i in range(k):
+        chain = (chain + A[:, i:i + 1].astype(np.float64) * B[i:i + 1].astype(np.float64)).astype(np.float32)
+    if k == 1:
+        np.testing.assert_array_equal(got, chain)
+    assert _rounding(got, A, B) <= 1.02 * _rounding(chain, A, B)
+
+
 @pytest.mark.parametrize("k", [100, 192, 4096])
 @pytest.mark.parametrize("sa,sb", [(1e-35, 1e20), (1e-37, 1e30), (1e-38, 1e30), (1e-40, 1e36), (1e-41, 1e37), (1e30, 1e-38), (1e36, 1e-40)])
 def test_operands_below_the_range_of_three_terms(on_hip, sa, sb, k):
