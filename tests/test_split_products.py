@@ -1,6 +1,8 @@
 """The matrix products and convolutions compute fp32 products from three bfloat16 terms per operand: rounding against float64 at the
 edges of the tiles, and what the three terms cannot hold (infinities, NaN, values that round up to infinity, values near the
 smallest normal one), which the kernels compute again with fp32 instructions."""
+import functools
+
 import numpy as np
 import pytest
 import torch
@@ -21,32 +23,6 @@ def _sgemm(be, ta, tb, A, B):
     return be.toHost(c, m * n).reshape(m, n)
 
 
-@pytest.mark.parametrize("tt", [(0, 0), (0, 1), (1, 0), (1, 1)])
-@pytest.mark.parametrize("dims", [(16, 64, 512), (64, 129, 257), (129, 128, 100), (333, 257, 31), (512, 640, 2048), (200, 136, 5000)])
-@pytest.mark.parametrize("spread", [0.0, 4.0])
-def test_products_against_float64(on_hip, tt, dims, spread):
-    """Per element: the six products of a group of 16 k are six roundings of the running sum (at most one unit, 2^-23, of its
-    size, which no partial sum's exceeds sum |a b|), a slice of a cut reduction (256 k and more) at most one more group and its
-    own addition, and the three products left out are below 3 * 2^-25 of |a b|."""
-    m, n, k = dims
-    rng = np.random.RandomState(7)
-    draw = lambda *s: (rng.standard_normal(s) * np.exp(spread * rng.standard_normal(s))).astype(np.float32)      # noqa: E731
-    A, B = draw(m, k), draw(k, n)
-    got = _sgemm(on_hip, tt[0], tt[1], A, B).astype(np.float64)
-    A64, B64 = A.astype(np.float64), B.astype(np.float64)
-    bound = (6 * -(-k // 16) + k // 32 + 2) * 2.0 ** -23 * (np.abs(A64) @ np.abs(B64))
-    assert (np.abs(got - A64 @ B64) <= bound).all()
-
-
-@pytest.mark.parametrize("scale", [1e-25, 1e-33, 1e-36])
-def test_products_of_tiny_values(on_hip, scale):
-    rng = np.random.RandomState(8)
-    A, B = (scale * rng.standard_normal((192, 192))).astype(np.float32), rng.standard_normal((192, 160)).astype(np.float32)
-    A64, B64 = A.astype(np.float64), B.astype(np.float64)
-    got = _sgemm(on_hip, 0, 0, A, B).astype(np.float64)
-    assert (np.abs(got - A64 @ B64) <= 192 * 2.0 ** -23 * (np.abs(A64) @ np.abs(B64))).all()
-
-
 # Root mean square of the error over sum |a b|.  Normal operands: rounding of a running sum of j terms is at most 2^-24 of its
 # size, sqrt(j); eight roundings per 16 k (the fp32 instructions) make 2^-24 / sqrt(3) * k / 2 over 2 / pi * k = 2.7e-8 at any
 # length, six (the three terms) 2.3e-8.  A row's figure, from 160 or 192 elements, stays within twice that.
@@ -56,6 +32,35 @@ ROUNDING = 2.0 * 2.7e-8
 def _rounding(got, A, B, axis=None):
     A64, B64 = A.astype(np.float64), B.astype(np.float64)
     return np.sqrt((((got.astype(np.float64) - A64 @ B64) / (np.abs(A64) @ np.abs(B64))) ** 2).mean(axis))
+
+
+@pytest.mark.parametrize("tt", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("dims", [(16, 64, 512), (64, 129, 257), (129, 128, 100), (333, 257, 31), (512, 640, 2048), (200, 136, 5000)])
+@pytest.mark.parametrize("spread", [0.0, 4.0])
+def test_products_against_float64(on_hip, tt, dims, spread):
+    """Per element: the six products of a group of 16 k are six roundings of the running sum (at most one unit, 2^-23, of its
+    size, which no partial sum's exceeds sum |a b|), a slice of a cut reduction (256 k and more) at most one more group and its
+    own addition, and the three products left out are below 3 * 2^-25 of |a b|.  Root mean square: no more than the fp32
+    instructions (2.7e-8 at any length for normal operands; of wide spread, 4.6e-7 measured at 8192 and less below), where any
+    one product more left out would be 5.4e-8 and more at these sizes (1.5e-6 and more for wide spread)."""
+    m, n, k = dims
+    rng = np.random.RandomState(7)
+    draw = lambda *s: (rng.standard_normal(s) * np.exp(spread * rng.standard_normal(s))).astype(np.float32)      # noqa: E731
+    A, B = draw(m, k), draw(k, n)
+    got = _sgemm(on_hip, tt[0], tt[1], A, B).astype(np.float64)
+    A64, B64 = A.astype(np.float64), B.astype(np.float64)
+    bound = (6 * -(-k // 16) + k // 32 + 2) * 2.0 ** -23 * (np.abs(A64) @ np.abs(B64))
+    assert (np.abs(got - A64 @ B64) <= bound).all()
+    assert _rounding(got, A, B) <= (2.8e-8 if spread == 0.0 else 4.6e-7)
+
+
+@pytest.mark.parametrize("scale", [1e-25, 1e-33, 1e-36])
+def test_products_of_tiny_values(on_hip, scale):
+    rng = np.random.RandomState(8)
+    A, B = (scale * rng.standard_normal((192, 192))).astype(np.float32), rng.standard_normal((192, 160)).astype(np.float32)
+    A64, B64 = A.astype(np.float64), B.astype(np.float64)
+    got = _sgemm(on_hip, 0, 0, A, B).astype(np.float64)
+    assert (np.abs(got - A64 @ B64) <= 192 * 2.0 ** -23 * (np.abs(A64) @ np.abs(B64))).all()
 
 
 @pytest.mark.parametrize("tt", [(0, 0), (0, 1), (1, 0), (1, 1)])
@@ -179,3 +184,90 @@ def test_plain_tile_plans_give_the_same_bits_around_what_the_terms_cannot_hold(o
     finally:
         monkeypatch.delenv("LH_FORCE_PLAN", raising=False)
         lib.lh_set_deterministic(0)
+
+
+REDO_SHAPES = [(4, 256, 14, 14, 256, 1, 1, 1, 1, 0, 0), (16, 128, 7, 7, 128, 3, 3, 1, 1, 1, 1), (8, 128, 28, 28, 96, 3, 3, 2, 2, 1, 1), (4, 24, 30, 26, 32, 5, 3, 2, 1, 0, 1)]
+
+
+@functools.lru_cache(maxsize=1)
+def _odd_convolution(dims):
+    """Inputs with an infinity, a NaN and a value below the range of the three terms in every 997th place; results and summed
+    magnitudes in float64 (forward, input gradient, filter gradient)."""
+    N, Cc, H, W, K, R, S, sH, sW, pH, pW = dims
+    P, Q = (H + 2 * pH - R) // sH + 1, (W + 2 * pW - S) // sW + 1
+    rng = np.random.RandomState(15)
+    x, w, dy = rng.randn(N, Cc, H, W).astype(np.float32), rng.randn(K, Cc, R, S).astype(np.float32), rng.randn(N, K, P, Q).astype(np.float32)
+    x.reshape(-1)[::997] = dy.reshape(-1)[::997] = w.reshape(-1)[::997] = 1.2345678e-39
+    x[1, 3, 4, 6] = dy[1, 3, 4, 5] = np.inf
+    x[N - 1, 2, H - 4, 0] = dy[N - 1, K - 1, P - 1, 0] = np.nan
+    conv = lambda a, b: torch.nn.functional.conv2d(a, b, stride=(sH, sW), padding=(pH, pW))      # noqa: E731
+
+    def all_three(x, w, dy):
+        xt, wt = (torch.from_numpy(a).double().requires_grad_() for a in (x, w))
+        y = conv(xt, wt)
+        return [y.detach().numpy()] + [g.numpy() for g in torch.autograd.grad(y, (xt, wt), torch.from_numpy(dy).double())]
+    clean = [np.abs(np.where(np.isfinite(a), a, 0)).astype(np.float32) for a in (x, w, dy)]
+    return x, w, dy, all_three(x, w, dy), all_three(*clean)
+
+
+def _check_odd(got, want, mag, what):
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want), err_msg=what)
+    np.testing.assert_array_equal(np.isinf(got), np.isinf(want), err_msg=what)
+    inf, ok = np.isinf(want), np.isfinite(want) & (mag > 0)
+    np.testing.assert_array_equal(got[inf], want[inf], err_msg=what)
+    err = np.abs(got[ok].astype(np.float64) - want[ok]) / mag[ok]
+    assert np.sqrt((err ** 2).mean()) <= ROUNDING, what
+    assert (got[np.isfinite(want) & (mag == 0)] == 0).all(), what
+
+
+@pytest.mark.parametrize("dims", REDO_SHAPES, ids=lambda d: "x".join(map(str, d)))
+@pytest.mark.parametrize("plan", [-1, 1, 2, 3, 4, 5, 6, 7, 8, 9, 11, 12, 13, 14, 15, "m32"])
+def test_what_the_terms_cannot_hold_under_every_launch_plan(on_hip, dims, plan, monkeypatch):
+    """Whole tiles, stream-K segments, sliced last tiles, the 32-row tile, the grouped launch of a strided input gradient, the filter
+    gradient's slices (added atomically and in order): infinities and NaN where float64 has them, the rest to rounding."""
+    x, w, dy, want, mag = _odd_convolution(dims)
+    dev, lib = Dev(on_hip), on_hip.lib
+    xd, wd, dyd = dev.up(x), dev.up(w), dev.up(dy)
+    if plan == "m32":
+        monkeypatch.setenv("LH_FORCE_M32", "1")
+    elif plan >= 0:
+        monkeypatch.setenv("LH_FORCE_PLAN", str(plan))
+    y, dx = dev.up(np.full(want[0].size, 7.0, np.float32)), dev.up(np.full(want[1].size, 7.0, np.float32))
+    lib.lh_conv2d_fwd(xd.ptr, wd.ptr, 0, y.ptr, *dims)
+    lib.lh_conv2d_bwd_data(dyd.ptr, wd.ptr, dx.ptr, 0.0, *dims)
+    dev.check()
+    _check_odd(dev.down(y, want[0].shape), want[0], mag[0], "forward")
+    _check_odd(dev.down(dx, want[1].shape), want[1], mag[1], "input gradient")
+    if plan in (-1, "m32"):
+        for deterministic in (0, 1):
+            lib.lh_set_deterministic(deterministic)
+            try:
+                dw = dev.up(np.full(want[2].size, 7.0, np.float32))
+                lib.lh_conv2d_bwd_filter(xd.ptr, dyd.ptr, dw.ptr, 0, 0.0, *dims)
+                dev.check()
+                _check_odd(dev.down(dw, want[2].shape), want[2], mag[2], "filter gradient, deterministic %d" % deterministic)
+            finally:
+                lib.lh_set_deterministic(0)
+
+
+@pytest.mark.parametrize("tile", [1, 2, 3, 5, 6, 7])
+def test_small_filter_rows_with_the_statistics_of_their_outputs(on_hip, tile, monkeypatch):
+    """The forward launch that leaves batch-norm statistics: filter rows below the range of the three terms against large inputs."""
+    dims = (6, 96, 15, 15, 160, 3, 3, 1, 1, 1, 1)
+    N, Cc, H, W, K = dims[:5]
+    rng = np.random.RandomState(16)
+    x, w = (1e10 * rng.randn(N, Cc, H, W)).astype(np.float32), 1e-10 * rng.randn(K, Cc, 3, 3)
+    w[5], w[70], w[159] = 1e-28 * w[5], 1e-30 * w[70], 1e-32 * w[159]
+    w = w.astype(np.float32)
+    want, mag = (torch.nn.functional.conv2d(*(torch.from_numpy(f(a).astype(np.float64)) for a in (x, w)), padding=1).numpy() for f in (np.array, np.abs))
+    dev, lib = Dev(on_hip), on_hip.lib
+    monkeypatch.setenv("LH_FORCE_STATS_TILE", str(tile))
+    xd, wd = dev.up(x), dev.up(w)
+    y, sm, si, rm, rv = dev.zeros(want.size), dev.zeros(K), dev.zeros(K), dev.zeros(K), dev.zeros(K)
+    lib.lh_conv2d_fwd_bnstats(xd.ptr, wd.ptr, 0, y.ptr, *dims, sm.ptr, si.ptr, rm.ptr, rv.ptr, 1e-5, 0.1)
+    dev.check()
+    err = (dev.down(y, want.shape).astype(np.float64) - want) / mag
+    assert (np.sqrt((err ** 2).mean((0, 2, 3))) <= ROUNDING).all()
+    # a channel's mean: 1350 sums, each off by at most a few units of its magnitudes
+    assert (np.abs(dev.down(sm, (K,)) - want.mean((0, 2, 3))) <= 1e-6 * mag.mean((0, 2, 3))).all()
+    assert (np.abs(dev.down(si, (K,)) * np.sqrt(want.var((0, 2, 3)) + 1e-5) - 1) <= 1e-5).all()
