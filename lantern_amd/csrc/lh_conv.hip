@@ -546,7 +546,7 @@ constexpr int CONV_BK = LH_CONV_BK;      // k-slab of the forward / input-gradie
 #ifndef LH_BWDF_BK
 #define LH_BWDF_BK 16
 #endif
-constexpr int BWDF_BK = LH_BWDF_BK;      // k-slab of the filter-gradient kernel
+constexpr int BWDF_BK = LH_BWDF_BK;      // k-slab of the filter-gradient kernel (32-row tiles: 32)
 // Forward / input-gradient launch.  A grid with few tiles per CU leaves CUs idle in its last wave
 // of blocks; such shapes run stream-K instead (largest tile, two workers per CU, every worker the
 // same number of k-slabs).  `zero_out`/`zero_n`: the output to clear first when the epilogue
@@ -1137,7 +1137,7 @@ void lh_conv2d_bwd_filter(const float* x, const float* dy, float* dw, float* db,
   float* partial = nullptr; size_t partial_bytes = 0; int slices = 1; bool on_side = false;
   // what igemm_launch will make of `split` for the tile in tp
   auto slices_of = [&](int sp) {
-    const int bk = tp.bm == 128 ? 16 : (tp.bm == 32 ? 32 : BWDF_BK);
+    const int bk = tp.bm == 32 ? 32 : BWDF_BK;
     int64_t kper = cdiv(cdiv(red, sp), bk) * bk; if (kper < bk) kper = bk;
     return (int)cdiv(red, kper);
   };
@@ -1147,7 +1147,7 @@ void lh_conv2d_bwd_filter(const float* x, const float* dy, float* dw, float* db,
     al.base = dy; al.nbytes = (uint32_t)((size_t)N * K * PQ * 4); al.K = K; al.PQ = PQ; al.dPQ.init(padded ? PQP : PQ);
     bl.base = x; bl.nbytes = (uint32_t)((size_t)N * C * H * W * 4); bl.C = C; bl.H = H; bl.W = W; bl.sH = sH; bl.sW = sW; bl.pH = pH; bl.pW = pW; bl.CHW = C * H * W;
     bl.P = d.P; bl.Q = d.Q; bl.dPQ.init(padded ? PQP : PQ); bl.dQ.init(d.Q); bl.dRS.init(R * S); bl.dS.init(S);
-    if (tp.bm == 128) ok = igemm_launch<128, 128, 16>(al, bl, ep, K, CRS, (int)red, split);    // measured: the large tile prefers the short slab
+    if (tp.bm == 128) ok = igemm_launch<128, 128, BWDF_BK>(al, bl, ep, K, CRS, (int)red, split);
     else if (tp.bm == 32) ok = igemm_launch<32, 128, 32>(al, bl, ep, K, CRS, (int)red, split);
     else if (tp.bn == 128) ok = igemm_launch<64, 128, BWDF_BK>(al, bl, ep, K, CRS, (int)red, split);
     else ok = igemm_launch<64, 64, BWDF_BK>(al, bl, ep, K, CRS, (int)red, split);
@@ -1156,7 +1156,7 @@ void lh_conv2d_bwd_filter(const float* x, const float* dy, float* dw, float* db,
   auto go_plain = [&](auto al, auto bl) {
     al.base = dy; al.nbytes = (uint32_t)((size_t)N * K * PQ * 4); al.K = K; al.PQ = PQ; al.dPQ.init(padded ? PQP : PQ);
     bl.base = x; bl.nbytes = (uint32_t)((size_t)N * C * PQ * 4); bl.K = C; bl.PQ = PQ; bl.dPQ.init(padded ? PQP : PQ);
-    if (tp.bm == 128) ok = igemm_launch<128, 128, 16>(al, bl, ep, K, CRS, (int)red, split);
+    if (tp.bm == 128) ok = igemm_launch<128, 128, BWDF_BK>(al, bl, ep, K, CRS, (int)red, split);
     else if (tp.bm == 32) ok = igemm_launch<32, 128, 32>(al, bl, ep, K, CRS, (int)red, split);
     else if (tp.bn == 128) ok = igemm_launch<64, 128, BWDF_BK>(al, bl, ep, K, CRS, (int)red, split);
     else ok = igemm_launch<64, 64, BWDF_BK>(al, bl, ep, K, CRS, (int)red, split);
