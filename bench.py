@@ -26,7 +26,7 @@ import numpy as np  # noqa: E402,F401
 
 # The products of fp32 operands run as six bfloat16 products each (three terms per operand, fp32 accumulation): a sixth of the
 # dense bfloat16 peak of 2516.6 TFLOP/s (the fp32 matrix instructions' own is 157.3).
-PEAK_FP32_MFMA_TFLOPS = 419.4
+PEAK_SPLIT_PRODUCTS_TFLOPS = 419.4
 PEAK_HBM_GBS = 8000.0
 # conv kernels of the headline step under rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE (profiles/resnet50_b64_hbm_traffic_and_mfma_counters.md)
 # 16.85 GB read + 7.98 GB written per step over 158 launches.  The measured launch plans decide how many launches a step has
@@ -339,8 +339,8 @@ def main():
         conv_t = sum(conv_ms) / 1000.0
         achieved = conv_fl / conv_t / 1e12 if conv_t > 0 else 0.0
         roof = {"bound": "mfma", "kernel": "k_igemm (conv fwd + bwd-data + bwd-filter, %d launches/step)" % conv_calls,
-                "achieved": round(achieved, 2), "peak": PEAK_FP32_MFMA_TFLOPS, "unit": "TFLOP/s",
-                "frac": round(achieved / PEAK_FP32_MFMA_TFLOPS, 4),
+                "achieved": round(achieved, 2), "peak": PEAK_SPLIT_PRODUCTS_TFLOPS, "unit": "TFLOP/s",
+                "frac": round(achieved / PEAK_SPLIT_PRODUCTS_TFLOPS, 4),
                 # HBM bytes per launch come from separate rocprofv3 FETCH_SIZE / WRITE_SIZE runs (profiles/), which this process cannot
                 # make: the profiled bytes of a step over THIS run's launches per step, and only when that count is within
                 # 5 % of the profiled run's (the same step, at most a few launches cut differently); otherwise null

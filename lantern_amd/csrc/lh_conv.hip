@@ -1,5 +1,5 @@
 // conv2D_batch forward, input gradient and filter gradient (NCHW fp32 cross-correlation) as
-// implicit GEMM on fp32 MFMA.  Reference behaviour being replaced: CPU:532-692 (im2col +
+// implicit GEMM on the matrix pipes (lh_igemm.h).  Reference behaviour being replaced: CPU:532-692 (im2col +
 // SGEMM per sample) and CDN:515-880 (cuDNN forward / backward-data / backward-filter / bias).
 //
 //   forward         Y[k, (n,p,q)]   = sum_{(c,r,s)} W[k, (c,r,s)]   * X[(c,r,s), (n,p,q)]
