@@ -15,6 +15,7 @@ extern hipStream_t g_stream_cur;
 void side_join();                 // the main stream waits for what the side stream was given (no-op when it is idle)
 void* persistent_alloc(size_t bytes);      // device memory of its own, outside the arena (waits for the device); nullptr when there is none
 void persistent_free(void* p);
+size_t arena_room();                       // bytes lh_malloc_uninit could hand out now
 bool side_work_begin();                    // library-internal fork: the side stream waits for the main stream and becomes current; false: not now
 void side_work_end();
 void build_filter_layout(int kind, const int* prm, const float* w, float* dst);      // lh_conv.hip: the copy kernel of a layout, on the current stream

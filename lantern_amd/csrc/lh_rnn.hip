@@ -5,12 +5,14 @@
 //   h_t = act(W_ih x_t + b_ih + W_hh h_{t-1} + b_hh),  h_{-1} = 0,   y[t,b,:] = [h_t forward ; h_t reverse]
 //
 // The input projection of all time steps and the three weight/input gradients are large GEMMs
-// (lh_sgemm, MFMA).  Only the recurrence is sequential: one small kernel per time step, both
+// (lh_sgemm, MFMA).  Only the recurrence is sequential: one launch for the whole sequence where its blocks fit the chip together
+// (lh_rnn_seq.hip), else, in the kernels of this file, one small launch per time step, both
 // directions in the same launch.  For aligned operands a block produces 16 hidden units for 16 batch rows
 // on the matrix pipes (lh_rnn_tile.h); otherwise 4-16 hidden units for the whole batch from W_hh rows held
 // in registers (the vector form).  The output y doubles as the saved hidden states.
 #include "lh_common.h"
 #include "lh_rnn_tile.h"
+#include "lh_rnn_seq.h"
 #include "../../include/lantern_hip.h"
 using namespace lh;
 
@@ -408,6 +410,20 @@ void lh_rnn_fwd_init(int mode, const float* x, const float* hx, const float* w, 
     if (hx) lh_sgemm(0, 1, B, H, H, 1.0f, hx + (size_t)d * B * H, H, Wih + (size_t)H * I, H, 1.0f, y + (size_t)(d == 0 ? 0 : T - 1) * B * ld + d * H, ld);
   }
   ProfScope prof_(CAT_RNN);
+  if (const size_t bytes = rnn_seq_scratch(SEQ_ELMAN, false, D, T, B, H)) {
+    SeqLayer a = {};
+    for (int d = 0; d < D; d++) {
+      a.dir[d].W = w + d * dir_params(I, H) + (size_t)H * I;
+      a.dir[d].b1 = a.dir[d].W + (size_t)H * H; a.dir[d].b2 = a.dir[d].b1 + H;
+    }
+    a.y = y; a.D = D; a.T = T; a.B = B; a.H = H; a.ld = ld; a.relu = mode == 0;
+    void* ring = lh_malloc_uninit(bytes);
+    if (ring == nullptr) return;
+    rnn_seq_run(SEQ_ELMAN, false, a, ring);
+    lh_free_top(bytes);
+    LH_CHECK_LAUNCH();
+    return;
+  }
   for (int step = 0; step < T; step++) {
     StepArgs a;
     for (int d = 0; d < 2; d++) {
@@ -441,11 +457,19 @@ void lh_rnn_bwd_init(int mode, const float* x, const float* hx, const float* y, 
   float* scratch = (float*)lh_malloc_uninit(bytes);
   if (scratch == nullptr) return;
   float* dpre = scratch; float* wt = dpre + n_dpre; float* colsum = wt + n_wt;
-  for (int d = 0; d < D; d++) {
-    const float* Whh = w + d * dir_params(I, H) + (size_t)H * I;
-    lh_trans(Whh, wt + (size_t)d * H * H, H, H);
-  }
-  {
+  if (const size_t ring_bytes = rnn_seq_scratch(SEQ_ELMAN, true, D, T, B, H)) {
+    SeqLayer a = {};
+    for (int d = 0; d < D; d++) a.dir[d].W = w + d * dir_params(I, H) + (size_t)H * I;
+    a.y = const_cast<float*>(y); a.dy = dy; a.dpre = dpre; a.D = D; a.T = T; a.B = B; a.H = H; a.ld = ld; a.relu = mode == 0;
+    void* ring = lh_malloc_uninit(ring_bytes);
+    if (ring == nullptr) return;
+    { ProfScope prof_(CAT_RNN); rnn_seq_run(SEQ_ELMAN, true, a, ring); }
+    lh_free_top(ring_bytes);
+  } else {
+    for (int d = 0; d < D; d++) {
+      const float* Whh = w + d * dir_params(I, H) + (size_t)H * I;
+      lh_trans(Whh, wt + (size_t)d * H * H, H, H);
+    }
     ProfScope prof_(CAT_RNN);
     // launch k produces dpre of the k-th slice in processing order (forward direction: t = T-1-k, reverse: t = k)
     for (int k = 0; k < T; k++) {

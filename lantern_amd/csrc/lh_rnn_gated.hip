@@ -7,13 +7,15 @@
 // b_hh[G] with G = 4H or 3H (NNModule.scala:378-390).
 //
 // Everything that is not sequential is one matrix product over all time steps (lh_sgemm on MFMA): the input projection,
-// both weight gradients, the input gradient.  A forward time step is one launch (the [B, H] x [H, G] product with the
+// both weight gradients, the input gradient.  The recurrence is one launch for the whole sequence where its blocks fit the chip
+// together (lh_rnn_seq.hip); otherwise a forward time step is one launch (the [B, H] x [H, G] product with the
 // previous state on 16 x 16 matrix tiles that hold all gates of four units, the gate arithmetic behind it); a backward
 // step, and a forward step on operands the tile kernel does not take, is a product plus one element-wise kernel over
 // [B, H].  The forward pass leaves the gate activations and the cell state (GRU: W_hn h + b_hn)
 // of every step in `reserve`; the backward pass turns the activations into pre-activation gradients in place.
 #include "lh_common.h"
 #include "lh_rnn_tile.h"
+#include "lh_rnn_seq.h"
 #include "../../include/lantern_hip.h"
 using namespace lh;
 
@@ -289,6 +291,25 @@ void lh_rnn_gated_fwd_init(int mode, const float* x, const float* hx, const floa
   const size_t gh_bytes = (size_t)D * per_dir * sizeof(float);
   float* gh_all = (float*)lh_malloc_uninit(gh_bytes);
   if (gh_all == nullptr) return;
+  if (const size_t ring_bytes = rnn_seq_scratch(mode == 2 ? SEQ_LSTM : SEQ_GRU, false, D, T, B, H)) {
+    SeqLayer s = {};
+    for (int d = 0; d < D; d++) {
+      SeqDir& p = s.dir[d];
+      const float* Wih = w + d * dir_params(mode, I, H);
+      p.W = Wih + (size_t)G * I; p.b1 = p.W + (size_t)G * H; p.b2 = p.b1 + G;
+      p.h0 = hx ? hx + (size_t)d * B * H : nullptr; p.c0 = cx ? cx + (size_t)d * B * H : nullptr;
+      p.act = reserve + d * dir_reserve(mode, T, B, H); p.aux = p.act + (size_t)T * B * G;
+      lh_sgemm(0, 1, T * B, G, I, 1.0f, x, I, Wih, I, 0.0f, p.act, G);
+    }
+    s.y = y; s.D = D; s.T = T; s.B = B; s.H = H; s.ld = ldh;
+    void* ring = lh_malloc_uninit(ring_bytes);
+    if (ring == nullptr) return;
+    rnn_seq_run(mode == 2 ? SEQ_LSTM : SEQ_GRU, false, s, ring);
+    lh_free_top(ring_bytes);
+    lh_free_top(gh_bytes);
+    LH_CHECK_LAUNCH();
+    return;
+  }
   // The two directions of a bidirectional layer share nothing but the input: the reverse one runs on the library's second
   // stream beside the forward one (in line when that stream is off, while a graph is recorded or in deterministic mode).
   auto run_direction = [&](int d) {
@@ -351,6 +372,22 @@ void lh_rnn_gated_bwd_init(int mode, const float* x, const float* hx, const floa
   const size_t bytes = (size_t)D * per_dir * sizeof(float);
   float* scratch = (float*)lh_malloc_uninit(bytes);
   if (scratch == nullptr) return;
+  const size_t ring_bytes = rnn_seq_scratch(mode == 2 ? SEQ_LSTM : SEQ_GRU, true, D, T, B, H);
+  if (ring_bytes) {
+    SeqLayer s = {};
+    for (int d = 0; d < D; d++) {
+      SeqDir& p = s.dir[d];
+      p.W = w + d * dir_params(mode, I, H) + (size_t)G * I;
+      p.h0 = hx ? hx + (size_t)d * B * H : nullptr; p.c0 = cx ? cx + (size_t)d * B * H : nullptr;
+      p.act = reserve + d * dir_reserve(mode, T, B, H); p.aux = p.act + (size_t)T * B * G;
+      p.dgh = scratch + (size_t)d * per_dir + 2 * n_bh + 2 * (size_t)G;
+    }
+    s.y = const_cast<float*>(y); s.dy = dy; s.D = D; s.T = T; s.B = B; s.H = H; s.ld = ldh;
+    void* ring = lh_malloc_uninit(ring_bytes);
+    if (ring == nullptr) return;
+    rnn_seq_run(mode == 2 ? SEQ_LSTM : SEQ_GRU, true, s, ring);
+    lh_free_top(ring_bytes);
+  }
   // each direction has its own scratch and its own part of dw, and runs on its own stream (see the forward pass); the input
   // gradient, to which both add, is formed afterwards on the caller's stream
   auto run_direction = [&](int d) {
@@ -360,7 +397,7 @@ void lh_rnn_gated_bwd_init(int mode, const float* x, const float* hx, const floa
     float* dWih = dw + off; float* dWhh = dWih + (size_t)G * I; float* dbih = dWhh + (size_t)G * H; float* dbhh = dbih + G;
     float* act = reserve + d * dir_reserve(mode, T, B, H);
     const float* aux = act + (size_t)T * B * G;
-    for (int k = 0; k < T; k++) {
+    for (int k = 0; k < T && !ring_bytes; k++) {
       const int t = d == 0 ? T - 1 - k : k;                        // reverse of the forward processing order
       const int tp = d == 0 ? t - 1 : t + 1;                       // the step whose state this one consumed
       const bool has_prev = d == 0 ? t > 0 : t < T - 1;

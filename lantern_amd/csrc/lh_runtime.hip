@@ -3,6 +3,7 @@
 // API:453-473 (myGpuMalloc / myGpuFree), CUB:37-107 (toGPU / toCPU).
 #include "lh_common.h"
 #include "lh_arena.h"
+#include "lh_rnn_seq.h"
 #include <stdarg.h>
 #include <string.h>
 #include <vector>
@@ -139,6 +140,7 @@ static void zero_async(void* p, size_t bytes) {  // bytes is a multiple of 256
   int grid = stream_grid((int64_t)n16, 256 * 4);
   hipLaunchKernelGGL(k_zero16, dim3(grid), dim3(256), 0, g_stream, (uint4*)p, n16);
 }
+size_t arena_room() { return g_arena.bytes - g_arena.top; }
 void zero_bytes_async(void* p, size_t bytes) { ProfScope prof_(CAT_FILL); zero_async(p, bytes); }
 }  // namespace lh
 using namespace lh;
@@ -173,6 +175,7 @@ void lh_setup(size_t heap_bytes) {
   LH_HIP(hipMalloc((void**)&g_fix_cnt, 4096 * sizeof(int)));          // FIX_MAX_TILES arrival counters (lh_igemm.h), zero between launches
   LH_HIP(hipMemset(g_fix_cnt, 0, 4096 * sizeof(int)));
   if (!multi_tensor_setup()) return;
+  if (!rnn_seq_setup()) return;
 }
 
 static void stage_release();
@@ -188,6 +191,7 @@ void lh_cleanup(void) {
   stage_release();
   copy_release();
   multi_tensor_release();
+  rnn_seq_release();
   for (auto& e : g_graphs) if (e) { (void)hipGraphExecDestroy(e); e = nullptr; }
   g_graphs.clear(); g_capturing = false;
   if (g_advance_pool) (void)hipFree(g_advance_pool);
@@ -205,6 +209,7 @@ void lh_sync(void) {
   side_join();
   lh_copy_join();
   LH_HIP(hipStreamSynchronize(g_stream)); LH_CHECK_LAUNCH();
+  (void)rnn_seq_report_timeout();
   (void)cmdlist_report_timeout();      // the wait is over: a barrier that gave up in a command-list launch is reported now, not at the next hand-over
 }
 
@@ -302,6 +307,7 @@ void lh_d2h(void* h_dst, const void* src, size_t bytes) {
   lh_copy_join();    // an upload still on the copy stream may be what is read back
   LH_HIP(hipMemcpyAsync(h_dst, src, bytes, hipMemcpyDeviceToHost, g_stream));
   LH_HIP(hipStreamSynchronize(g_stream));
+  (void)rnn_seq_report_timeout();
   (void)cmdlist_report_timeout();
 }
 // ---- transfers that do not stall the step: pinned host memory, a copy stream for uploads, read-backs without a wait ----
