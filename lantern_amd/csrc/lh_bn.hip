@@ -5,6 +5,7 @@
 // partial statistics go through a small device scratch and are combined (Chan's parallel
 // variance formula, in double) by every block of the second pass.
 #include "lh_common.h"
+#include "lh_infer.h"
 using namespace lh;
 
 namespace {
@@ -348,12 +349,43 @@ __global__ void __launch_bounds__(TPB) k_bn_small_bwd_join(const float* __restri
   }
 }
 
-__global__ void __launch_bounds__(TPB) k_bn_infer(const float* __restrict__ x, float* __restrict__ y, const float* gamma, const float* beta,
-                                                  const float* rmean, const float* rvar, int C, int HW, int64_t n, float eps) {
-  int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x, st = (int64_t)gridDim.x * TPB;
-  for (; i < n; i += st) {
-    int c = (int)((i / HW) % C);
-    y[i] = (x[i] - rmean[c]) / sqrtf(rvar[c] + eps) * gamma[c] + beta[c];
+// Running statistics: y = act((x - mean) * (gamma / sqrt(var + eps)) + beta [+ shortcut]), the convolution epilogue's formula
+// (EpiConvBn): the factor of a channel is formed once, not a square root and a division per element.
+__device__ __forceinline__ float bn_infer_value(float x, float m, float s, float b) { return fmaf(x - m, s, b); }
+// a block: a run of 4 * TPB elements of one channel image (VEC: HW % 4 == 0, aligned operands)
+template <bool VEC, bool ADD, bool RELU>
+__global__ void __launch_bounds__(TPB) k_bn_infer(const float* x, float* y, const float* __restrict__ shortcut, const float* __restrict__ gamma, const float* __restrict__ beta,
+                                                  const float* __restrict__ mean, const float* __restrict__ var, int C, int HW, int runs, float eps) {
+  const int img = blockIdx.x / runs, run = blockIdx.x - img * runs, c = img % C;
+  const float m = mean[c], b = beta[c], s = gamma[c] / sqrtf(var[c] + eps);
+  const int64_t base = (int64_t)img * HW;
+  auto one = [&](float v, float a) { float r = bn_infer_value(v, m, s, b); if (ADD) r += a; if (RELU) r = r < 0.f ? 0.f : r; return r; };
+  if (VEC) {
+    const int i = (run * TPB + (int)threadIdx.x) * 4;
+    if (i < HW) {
+      const float4 v = *reinterpret_cast<const float4*>(x + base + i);
+      float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (ADD) a = *reinterpret_cast<const float4*>(shortcut + base + i);
+      *reinterpret_cast<float4*>(y + base + i) = make_float4(one(v.x, a.x), one(v.y, a.y), one(v.z, a.z), one(v.w, a.w));
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int i = run * 4 * TPB + q * TPB + (int)threadIdx.x;
+      if (i < HW) y[base + i] = one(x[base + i], ADD ? shortcut[base + i] : 0.f);
+    }
+  }
+}
+// small images (HW below a block): consecutive elements over the threads
+template <bool ADD, bool RELU>
+__global__ void __launch_bounds__(TPB) k_bn_infer_small(const float* x, float* y, const float* __restrict__ shortcut, const float* __restrict__ gamma, const float* __restrict__ beta,
+                                                        const float* __restrict__ mean, const float* __restrict__ var, int C, int HW, int64_t n, float eps) {
+  for (int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x; i < n; i += (int64_t)gridDim.x * TPB) {
+    const int c = (int)((i / HW) % C);
+    float r = bn_infer_value(x[i], mean[c], gamma[c] / sqrtf(var[c] + eps), beta[c]);
+    if (ADD) r += shortcut[i];
+    if (RELU) r = r < 0.f ? 0.f : r;
+    y[i] = r;
   }
 }
 
@@ -717,16 +749,42 @@ void lh_bn_apply(const float* x, const float* gamma, const float* beta, const fl
   LH_CHECK_LAUNCH();
 }
 
+}  // extern "C"
+namespace lh {
+void bn_infer_now(const float* x, const float* gamma, const float* beta, const float* mean, const float* var, float eps, const float* shortcut, float* y,
+                  int relu, int N, int C, int HW) {
+  const int64_t n = (int64_t)N * C * HW;
+  if (n <= 0) return;
+  ProfScope prof_(CAT_BN_FWD);
+  work_add(CAT_BN_FWD, (shortcut ? 12.0 : 8.0) * (double)n);
+  const bool vec = HW % 4 == 0 && (((uintptr_t)x | (uintptr_t)y | (uintptr_t)shortcut) & 15) == 0;
+  const int64_t runs = cdiv(HW, 4 * TPB), blocks = runs * N * C;
+  if (HW < TPB || blocks > 0x7fffffff) {
+#define GO(A, R) hipLaunchKernelGGL((k_bn_infer_small<A, R>), dim3(stream_grid(n, TPB * 4)), dim3(TPB), 0, g_stream, x, y, shortcut, gamma, beta, mean, var, C, HW, n, eps)
+    if (shortcut) { if (relu) GO(true, true); else GO(true, false); } else { if (relu) GO(false, true); else GO(false, false); }
+#undef GO
+  } else {
+#define GO(V, A, R) hipLaunchKernelGGL((k_bn_infer<V, A, R>), dim3((unsigned)blocks), dim3(TPB), 0, g_stream, x, y, shortcut, gamma, beta, mean, var, C, HW, (int)runs, eps)
+#define GO2(A, R) do { if (vec) GO(true, A, R); else GO(false, A, R); } while (0)
+    if (shortcut) { if (relu) GO2(true, true); else GO2(true, false); } else { if (relu) GO2(false, true); else GO2(false, false); }
+#undef GO2
+#undef GO
+  }
+  LH_CHECK_LAUNCH();
+}
+}  // namespace lh
+extern "C" {
+
 void lh_bn_infer(const float* x, const float* gamma, const float* beta, const float* run_mean, const float* run_var,
                  float* y, int N, int C, int HW, float eps) {
   int64_t n = (int64_t)N * C * HW;
   if (n <= 0) return;
-  LZ_ENTER(); lazy::rd_f(x, n); lazy::rd_f(gamma, C); lazy::rd_f(beta, C); lazy::rd_f(run_mean, C); lazy::rd_f(run_var, C);
+  LZ_SCOPE();
+  if (lazy::park_bn_infer(x, gamma, beta, run_mean, run_var, y, N, C, HW, eps)) return;       // right behind a convolution: its epilogue does it
+  if (lazy::g_busy && !lazy::g_replay) lazy::flush_parked();
+  lazy::rd_f(x, n); lazy::rd_f(gamma, C); lazy::rd_f(beta, C); lazy::rd_f(run_mean, C); lazy::rd_f(run_var, C);
   lazy::out_f(y, n, y == x);
-  ProfScope prof_(CAT_BN_FWD);
-  work_add(CAT_BN_FWD, 8.0 * (double)n);
-  hipLaunchKernelGGL(k_bn_infer, dim3(stream_grid(n, TPB * 4)), dim3(TPB), 0, g_stream, x, y, gamma, beta, run_mean, run_var, C, HW, n, eps);
-  LH_CHECK_LAUNCH();
+  bn_infer_now(x, gamma, beta, run_mean, run_var, eps, nullptr, y, 0, N, C, HW);
 }
 
 static void bn_train_fwd_impl(bool relu, const float* x, const float* gamma, const float* beta, float* run_mean, float* run_var, float* y,

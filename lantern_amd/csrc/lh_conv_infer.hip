@@ -1,0 +1,123 @@
+// Forward convolution with a batch norm on running statistics, the residual join and relu in its epilogue: what the deferred work
+// (lh_defer.hip) makes of conv2D_batch -> batchNormInference [-> + shortcut] [-> relu in place], the calls of a network that is
+// served (the reference's readONNX inference_func, src/main/scala/lantern/ONNXLib.scala:597-830).
+#include "lh_conv_fwd.h"
+#include "lh_infer.h"
+using namespace lh;
+
+namespace {
+// y = act((v - mean) * (gamma / sqrt(var + eps)) + beta [+ shortcut]) with v = sum + bias: k_bn_infer's formula, operation by
+// operation, so that the chain gives the bits of its parts.  Complete sums only (no stream-K).
+struct EpiConvBn : EpiConvOut {
+  static constexpr bool ROWS = true;
+  const float* gamma; const float* shift; const float* mean; const float* var; float eps;
+  const float* shortcut;
+  __device__ __forceinline__ float4 row_params(int row, int M) const {
+    if (row >= M) return make_float4(0.f, 0.f, 0.f, 0.f);
+    return make_float4(mean[row], gamma[row] / sqrtf(var[row] + eps), shift[row], bias ? bias[row] : 0.f);
+  }
+  __device__ __forceinline__ float row_value(float v, const float4 p, float other, bool join) const {
+    if (bias) v += p.w;
+    float r = fmaf(v - p.x, p.y, p.z);
+    if (join) r += other;
+    if (relu) r = r < 0.f ? 0.f : r;
+    return r;
+  }
+  __device__ __forceinline__ int lean_mode() const { return shortcut ? 3 : 0; }
+  __device__ __forceinline__ const float* lean_other() const { return shortcut; }
+  __device__ __forceinline__ void store_row(const Col& c, int i, int M, float v, const float4 p) const {
+    if (!c.valid || i >= M) return;
+    const int64_t at = (int64_t)c.off + (int64_t)i * PIX;
+    out[at] = row_value(v, p, shortcut ? shortcut[at] : 0.f, shortcut != nullptr);
+  }
+};
+
+// Launch forms: 1-3 whole tiles 128x128, 64x128, 64x64; 5-7 the last tiles of 64x64 / 64x128 / 128x128 sliced along the reduction
+// (igemm_launch_shared_tail); 4 the convolution by itself (any of its launch plans, stream-K among them), then the pass over it.
+template <class AL, class BL>
+bool launch_form(int form, const AL& al, const BL& bl, const EpiConvBn& ep, int M, int N, int K) {
+  if (form == 1) return igemm_launch<128, 128, CONV_BK>(al, bl, ep, M, N, K, 1);
+  if (form == 2) return igemm_launch<64, 128, CONV_BK>(al, bl, ep, M, N, K, 1);
+  if (form == 5) return igemm_launch_shared_tail<64, 64, CONV_BK>(al, bl, ep, M, N, K);
+  if (form == 6) return igemm_launch_shared_tail<64, 128, CONV_BK>(al, bl, ep, M, N, K);
+  if (form == 7) return igemm_launch_shared_tail<128, 128, CONV_BK>(al, bl, ep, M, N, K);
+  return igemm_launch<64, 64, CONV_BK>(al, bl, ep, M, N, K, 1);
+}
+int form_of_rule(int M, int N, int K) {
+  const TilePick tp = pick_tile_conv(M, N, K);
+  return tp.bm == 128 ? 1 : (tp.bn == 128 ? 2 : 3);
+}
+}  // namespace
+
+namespace lh {
+// ResNet-50 at 224x224 on one card in turn, 53 such chains (before: 53 convolutions, 53 batch norms, 33 relus and 16 joins, each a pass
+// over memory): batch 32 4.28 -> 2.90 ms, batch 1 1.006 -> 0.797 ms.  What bounds it now is the convolutions themselves.
+void conv2d_bn_infer_now(const float* x, const float* w, const float* bias, int N, int C, int H, int W, int K, int R, int S, int sH, int sW, int pH, int pW,
+                         const float* gamma, const float* beta, const float* mean, const float* var, float eps, const float* shortcut, float* out, int relu) {
+  KernelCat kc_(CAT_CONV_FWD);
+  ConvDims d;
+  LH_REQUIRE(make_dims(d, N, C, H, W, K, R, S, sH, sW, pH, pW), "lh_conv2d_fwd: bad shape N%d C%d H%d W%d K%d R%d S%d s(%d,%d) p(%d,%d)", N, C, H, W, K, R, S, sH, sW, pH, pW);
+  const int RS = R * S, CRS = C * RS, PQ = d.P * d.Q, cols = N * PQ;
+  const uint32_t wbytes = (uint32_t)((size_t)K * CRS * 4), xbytes = (uint32_t)((size_t)N * C * H * W * 4);
+  EpiConvBn ep;
+  static_cast<EpiConvOut&>(ep) = make_epi(out, bias, K, d.P, d.Q, 0.f);
+  ep.relu = relu; ep.gamma = gamma; ep.shift = beta; ep.mean = mean; ep.var = var; ep.eps = eps; ep.shortcut = shortcut;
+  bool ok;
+  if (C % CONV_BK == 0 && ((uintptr_t)w & 15) == 0) {
+    // tap-major reduction order; a 1x1 filter already has that layout
+    FilterCopy fc;
+    fc.p = const_cast<float*>(w);
+    const int prm[LAYOUT_PRM] = {K, C, RS};
+    if (RS > 1 && !filter_copy(fc, w, wbytes, LAYOUT_KRSC, prm, wbytes)) return;
+    LoadPlainK<true> al; al.base = fc.p; al.nbytes = wbytes; al.ld = CRS;
+    LoadConvFwdTapB bl; bl.base = x; bl.nbytes = xbytes; bl.C = C; bl.H = H; bl.W = W; bl.sH = sH; bl.sW = sW; bl.pH = pH; bl.pW = pW; bl.HW = H * W;
+    bl.dPQ.init(PQ); bl.dQ.init(d.Q); bl.dC.init(C); bl.dS.init(S);
+    auto run = [&](int form) {
+      if (form != 4) return launch_form(form, al, bl, ep, K, cols, CRS);
+      lh_conv2d_fwd(x, w, bias, out, N, C, H, W, K, R, S, sH, sW, pH, pW);
+      if (!failed()) bn_infer_now(out, gamma, beta, mean, var, eps, shortcut, out, relu, N, K, PQ);
+      return !failed();
+    };
+    auto valid = [&](int form) {
+      if ((form == 1 || form == 7) && K <= 64) return false;
+      if (form >= 5) return !g_deterministic && g_stream_cur == g_stream_raw && CRS >= 8 * CONV_BK;
+      // the convolution by itself: where its tiles are fewer than the compute units and the reduction is long enough for stream-K
+      if (form == 4) return !g_deterministic && cdiv(K, 64) * cdiv(cols, 64) < g_num_cu && CRS >= 16 * CONV_BK;
+      return true;
+    };
+    // the form is measured once per shape (the launch overwrites `out` and nothing else, so repeating it is harmless) and remembered
+    static std::map<PlanKey, int> chosen;
+    const PlanKey key = {{K, cols, CRS, H, W, sH, R | (shortcut ? 1 << 16 : 0) | (g_deterministic ? 1 << 17 : 0)}};
+    int form = form_of_rule(K, cols, CRS);
+    const int forced = force_plan() >= 13 && force_plan() <= 15 ? force_plan() - 8 : force_plan();
+    auto it = chosen.find(key);
+    if (forced >= 1 && forced <= 7 && valid(forced)) form = forced;
+    else if (it != chosen.end() && g_tune_enabled) { form = it->second; g_plans_remembered++; }
+    else if (g_tune_enabled && !g_capturing && 2.0 * K * CRS * (double)cols >= g_tune_min_flop) {
+      LaunchTimer timer;
+      if (timer.ok) {
+        float best_ms = 3.0e38f;
+        const int order[7] = {3, 2, 1, 5, 6, 7, 4};
+        for (int f : order) {
+          if (!valid(f)) continue;
+          const float ms = timer.ms([&]() { return run(f); });
+          if (ms < 0.f || failed()) { if (fc.scratch) lh_free_top(fc.scratch); return; }
+          if (ms < best_ms * 0.98f) { best_ms = ms; form = f; }
+        }
+        chosen[key] = form; g_plans_measured++;
+        if (getenv("LH_TUNE_VERBOSE")) fprintf(stderr, "conv + bn (running) K%d N%d CRS%d H%d: form %d, %.4f ms\n", K, cols, CRS, H, form, best_ms);
+      }
+    }
+    ok = run(form);
+    if (fc.scratch) lh_free_top(fc.scratch);
+  } else {
+    LoadConvFwdB bl; bl.base = x; bl.nbytes = xbytes; bl.C = C; bl.H = H; bl.W = W; bl.sH = sH; bl.sW = sW; bl.pH = pH; bl.pW = pW; bl.HW = H * W;
+    bl.dPQ.init(PQ); bl.dQ.init(d.Q); bl.dRS.init(RS); bl.dS.init(S);
+    LoadPlainK<false> al; al.base = w; al.nbytes = wbytes; al.ld = CRS;
+    if (form_of_rule(K, cols, CRS) == 3) ok = igemm_launch<64, 64, CONV_BK>(al, bl, ep, K, cols, CRS, 1);
+    else ok = igemm_launch<64, 128, CONV_BK>(al, bl, ep, K, cols, CRS, 1);
+  }
+  if (!ok) return;
+  LH_CHECK_LAUNCH();
+}
+}  // namespace lh

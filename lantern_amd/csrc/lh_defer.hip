@@ -25,6 +25,7 @@
 // Apart from the memory of the filter copies (allocated when a filter is first seen, released with it), nothing here
 // allocates device memory or waits for the device.
 #include "lh_common.h"
+#include "lh_infer.h"
 #include <string.h>
 #include <algorithm>
 #include <vector>
@@ -47,19 +48,20 @@ static inline bool covers(const char* a, size_t an, const char* b, size_t bn) { 
 struct ZeroBlock { char* p; size_t bytes; };
 static std::vector<ZeroBlock> g_zero;          // ascending addresses: the arena is a bump allocator
 
-enum { V_MASK = 0, V_BN_OUT = 1 };
+enum { V_MASK = 0, V_BN_OUT = 1, V_CONV = 2, V_BN_INFER = 3 };
+struct ConvArgs { const float* x; const float* w; const float* bias; float* y; int N, C, H, W, K, R, S, sH, sW, pH, pW, P, Q; };
 struct Unwritten {
   int kind; char* dst; size_t bytes;
   const float* src; const float* y; int64_t n;                                           // V_MASK: dst = y > 0 ? src : 0
-  const float* x; const float* gamma; const float* beta; const float* sm; const float* si; int N, C, HW;   // V_BN_OUT: dst = bn(x)
+  const float* x; const float* gamma; const float* beta; const float* sm; const float* si; int N, C, HW;   // V_BN_OUT: dst = bn(x); V_BN_INFER: the same from running statistics (sm, si: mean, variance)
+  float eps; ConvArgs conv;                                                              // V_CONV: dst = conv(x)
 };
 static std::vector<Unwritten> g_unwritten;
 
 struct FwdRecord { const float* y; const float* x; const float* bias; int64_t n; };   // y = relu(bn(x)) as the fused kernels compute it
 static std::vector<FwdRecord> g_records;
 
-struct ConvArgs { const float* x; const float* w; const float* bias; float* y; int N, C, H, W, K, R, S, sH, sW, pH, pW, P, Q; };
-struct BnArgs { const float* x; const float* gamma; const float* beta; float* rm; float* rv; float* y; float* sm; float* si; int N, C, HW; float eps, factor; int64_t n; };
+struct BnArgs { const float* x; const float* gamma; const float* beta; float* rm; float* rv; float* y; float* sm; float* si; int N, C, HW; float eps, factor; int64_t n; bool infer = false; };
 struct AddArgs { const float* a; const float* b; float* out; int64_t n; };
 enum { P_NONE = 0, P_CONV, P_BN, P_ADD, P_RELU_GRAD, P_RELU_ADD_GRAD, P_UPDATE };
 struct Parked {
@@ -193,20 +195,37 @@ static void clear_blocks(size_t first, size_t last) {
 static void produce(const Unwritten& v) {
   // what the recipe reads may itself be deferred
   if (v.kind == V_MASK) { rd(v.src, (size_t)v.n * 4); rd(v.y, (size_t)v.n * 4); }
+  else if (v.kind == V_CONV) { const ConvArgs& c = v.conv; rd(c.x, (size_t)c.N * c.C * c.H * c.W * 4); rd(c.w, (size_t)c.K * c.C * c.R * c.S * 4); if (c.bias) rd(c.bias, (size_t)c.K * 4); }
   else { rd(v.x, (size_t)v.n * 4); }
   Replay r_;
   g_stat[ST_RECIPES]++;
+  const ConvArgs& c = v.conv;
   if (v.kind == V_MASK) mask_relu((float*)v.dst, v.src, v.y, v.n);
+  else if (v.kind == V_CONV) lh_conv2d_fwd(c.x, c.w, c.bias, c.y, c.N, c.C, c.H, c.W, c.K, c.R, c.S, c.sH, c.sW, c.pH, c.pW);
+  else if (v.kind == V_BN_INFER) bn_infer_now(v.x, v.gamma, v.beta, v.sm, v.si, v.eps, nullptr, (float*)v.dst, 0, v.N, v.C, v.HW);
   else lh_bn_apply(v.x, v.gamma, v.beta, v.sm, v.si, (float*)v.dst, v.N, v.C, v.HW, 0);
 }
 static bool reads(const Unwritten& v, const char* lo, size_t nb) {
   if (v.kind == V_MASK) return overlap(lo, nb, (const char*)v.src, (size_t)v.n * 4) || overlap(lo, nb, (const char*)v.y, (size_t)v.n * 4);
+  if (v.kind == V_CONV) {
+    const ConvArgs& c = v.conv;
+    return overlap(lo, nb, (const char*)c.x, (size_t)c.N * c.C * c.H * c.W * 4) || overlap(lo, nb, (const char*)c.w, (size_t)c.K * c.C * c.R * c.S * 4) ||
+           (c.bias && overlap(lo, nb, (const char*)c.bias, (size_t)c.K * 4));
+  }
   const size_t cb = (size_t)v.C * 4;
   return overlap(lo, nb, (const char*)v.x, (size_t)v.n * 4) || overlap(lo, nb, (const char*)v.gamma, cb) || overlap(lo, nb, (const char*)v.beta, cb) ||
          overlap(lo, nb, (const char*)v.sm, cb) || overlap(lo, nb, (const char*)v.si, cb);
 }
 // mode 0: the range is read; 1: overwritten as a whole; 2: read and written
 static void settle_unwritten(const char* lo, size_t nb, int mode) {
+  // a batch norm's output whose recipe reads an output that is unwritten itself goes first: dropping that one (it is about to be
+  // overwritten) would leave the recipe nothing to read
+  if (mode != 0)
+    for (size_t i = 0; i < g_unwritten.size();) {
+      const Unwritten& v = g_unwritten[i];
+      if (v.kind == V_BN_INFER && reads(v, lo, nb) && !covers(lo, round256(nb), v.dst, v.bytes)) { const Unwritten copy = v; g_unwritten.erase(g_unwritten.begin() + i); produce(copy); i = 0; }
+      else i++;
+    }
   for (size_t i = 0; i < g_unwritten.size();) {
     const Unwritten& v = g_unwritten[i];
     const bool hit_dst = overlap(lo, nb, v.dst, v.bytes);
@@ -232,7 +251,6 @@ void rd(const void* p, size_t bytes) {
 void wr(const void* p, size_t bytes) {
   if (!g_busy || g_replay || p == nullptr || bytes == 0) return;
   const char* lo = (const char*)p;
-  layouts_written(lo, bytes);
   size_t a, b; zero_span(lo, lo + bytes, a, b);
   // blocks the write covers need no clearing; a block it only touches is cleared first
   while (a < b) {
@@ -240,29 +258,31 @@ void wr(const void* p, size_t bytes) {
     else { clear_blocks(a, a + 1); b--; }
   }
   if (!g_unwritten.empty()) settle_unwritten(lo, bytes, 1);
+  layouts_written(lo, bytes);         // (behind the recipes: one that reads this filter may have made its copy again)
   refresh_busy();
 }
 void rw(const void* p, size_t bytes) {
   if (!g_busy || g_replay || p == nullptr || bytes == 0) return;
   const char* lo = (const char*)p;
-  layouts_written(lo, bytes);
   size_t a, b; zero_span(lo, lo + bytes, a, b); clear_blocks(a, b);
   if (!g_unwritten.empty()) settle_unwritten(lo, bytes, 2);
+  layouts_written(lo, bytes);
   refresh_busy();
 }
 bool acc(const void* p, size_t bytes) {
   if (!g_busy || g_replay || p == nullptr || bytes == 0) return false;
   const char* lo = (const char*)p;
-  layouts_written(lo, bytes);
   size_t a, b; zero_span(lo, lo + bytes, a, b);
   if (b == a + 1 && g_zero[a].p == lo && g_zero[a].bytes == round256(bytes)) {       // the whole block, still untouched: overwrite it
     g_zero.erase(g_zero.begin() + a);
     g_stat[ST_ZERO_SKIPPED]++;
+    layouts_written(lo, bytes);
     refresh_busy();
     return true;
   }
   clear_blocks(a, b);
   if (!g_unwritten.empty()) settle_unwritten(lo, bytes, 2);
+  layouts_written(lo, bytes);
   refresh_busy();
   return false;
 }
@@ -283,6 +303,23 @@ static void launch_bn_chain(const Parked& p, int relu, const float* shortcut, fl
     lh_bn_train_fwd(b.x, b.gamma, b.beta, b.rm, b.rv, out, b.sm, b.si, b.N, b.C, b.HW, b.eps, b.factor);
   }
 }
+// The inference chain: one launch leaves out what nobody normally reads, the convolution's output and, under a join, the batch
+// norm's; both are noted with their recipes.
+static void launch_infer_chain(const Parked& p, int relu, const float* shortcut, float* out) {
+  const ConvArgs& c = p.conv; const BnArgs& b = p.bn;
+  {
+    Replay r_;
+    conv2d_bn_infer_now(c.x, c.w, c.bias, c.N, c.C, c.H, c.W, c.K, c.R, c.S, c.sH, c.sW, c.pH, c.pW, b.gamma, b.beta, b.rm, b.rv, b.eps, shortcut, out, relu);
+  }
+  Unwritten v{}; v.kind = V_CONV; v.dst = (char*)c.y; v.bytes = (size_t)b.n * 4; v.n = b.n; v.conv = c;
+  g_unwritten.push_back(v);
+  if (shortcut) {
+    Unwritten u{}; u.kind = V_BN_INFER; u.dst = (char*)b.y; u.bytes = (size_t)b.n * 4; u.n = b.n;
+    u.x = b.x; u.gamma = b.gamma; u.beta = b.beta; u.sm = b.rm; u.si = b.rv; u.eps = b.eps; u.N = b.N; u.C = b.C; u.HW = b.HW;
+    g_unwritten.push_back(u);
+  }
+  g_stat[ST_FUSED_FWD]++;
+}
 static void note_mask(float* dst, const float* src, const float* y, int64_t n) {
   Unwritten v{}; v.kind = V_MASK; v.dst = (char*)dst; v.bytes = (size_t)n * 4; v.src = src; v.y = y; v.n = n;
   g_unwritten.push_back(v);
@@ -292,6 +329,11 @@ void flush_parked() {
   if (g_p.kind == P_NONE) return;
   Parked p = std::move(g_p);
   g_p = Parked();
+  if (p.kind == P_BN && p.bn.infer) {
+    launch_infer_chain(p, 0, p.has_add ? (p.bn.y == p.add.a ? p.add.b : p.add.a) : nullptr, p.has_add ? p.add.out : p.bn.y);
+    refresh_busy();
+    return;
+  }
   if (p.kind == P_UPDATE) {
     // stated now, not when the calls were gathered: a rewind in between has released what depended on the old parameter values
     for (size_t i = 0; i < p.ux.size(); i++) {
@@ -377,12 +419,41 @@ bool park_bn_train_fwd(const float* x, const float* gamma, const float* beta, fl
   return true;
 }
 
+// Batch norm with running statistics right behind a parked convolution.  (Not while a graph is recorded: whatever is unread when the
+// recording ends is produced in it, and the graph would run every convolution twice.)  The fused launch writes the batch norm's
+// output, or the join's, while it reads the convolution's operands: outputs that lie over any of those run as issued.
+static bool over_conv_operands(const ConvArgs& c, const float* p, int64_t n) {
+  const char* lo = (const char*)p; const size_t nb = (size_t)n * 4;
+  return overlap(lo, nb, (const char*)c.x, (size_t)c.N * c.C * c.H * c.W * 4) || overlap(lo, nb, (const char*)c.w, (size_t)c.K * c.C * c.R * c.S * 4) ||
+         overlap(lo, nb, (const char*)c.y, (size_t)c.N * c.K * c.P * c.Q * 4) || (c.bias && overlap(lo, nb, (const char*)c.bias, (size_t)c.K * 4));
+}
+static bool over_channels(const BnArgs& b, const float* p, int64_t n) {
+  for (const float* q : {b.gamma, b.beta, (const float*)b.rm, (const float*)b.rv}) if (overlap((const char*)p, (size_t)n * 4, (const char*)q, (size_t)b.C * 4)) return true;
+  return false;
+}
+bool park_bn_infer(const float* x, const float* gamma, const float* beta, const float* mean, const float* var, float* y, int N, int C, int HW, float eps) {
+  if (!can_park() || g_capturing || conv2d_bn_infer_now == nullptr || bn_infer_now == nullptr || !x || !gamma || !beta || !mean || !var || !y) return false;
+  const int64_t n = (int64_t)N * C * HW;
+  if (!(g_p.kind == P_CONV && g_p.conv.y == x && g_p.conv.N == N && g_p.conv.K == C && (int64_t)g_p.conv.P * g_p.conv.Q == HW)) return false;
+  BnArgs b = {x, gamma, beta, const_cast<float*>(mean), const_cast<float*>(var), y, nullptr, nullptr, N, C, HW, eps, 0.f, n};
+  b.infer = true;
+  if (over_conv_operands(g_p.conv, y, n) || over_channels(b, y, n)) return false;
+  for (const float* q : {gamma, beta, mean, var}) if (overlap((const char*)q, (size_t)C * 4, (const char*)x, (size_t)n * 4)) return false;
+  rd(gamma, (size_t)C * 4); rd(beta, (size_t)C * 4); rd(mean, (size_t)C * 4); rd(var, (size_t)C * 4);
+  wr(y, (size_t)n * 4);
+  g_p.kind = P_BN; g_p.has_add = false; g_p.bn = b;
+  g_busy = true;
+  return true;
+}
+
 bool park_add(const float* a, const float* b, float* out, int64_t n) {
   if (!can_park() || !a || !b || !out || n <= 0 || out == a || out == b) return false;
   if (g_p.kind == P_BN && !g_p.has_add && a != b && n == g_p.bn.n && (g_p.bn.y == a || g_p.bn.y == b)) {
     const float* other = g_p.bn.y == a ? b : a;
     // relu(bn(h) + h): the fused backward would have one buffer for both of its gradients; that join stays unfused
-    if (other != g_p.bn.x && !overlap((const char*)other, (size_t)n * 4, (const char*)out, (size_t)n * 4)) {
+    const bool clear = !g_p.bn.infer || !(over_conv_operands(g_p.conv, out, n) || over_channels(g_p.bn, out, n) || overlap((const char*)other, (size_t)n * 4, (const char*)g_p.conv.y, (size_t)n * 4) ||
+                                          overlap((const char*)other, (size_t)n * 4, (const char*)g_p.bn.y, (size_t)n * 4) || overlap((const char*)out, (size_t)n * 4, (const char*)g_p.bn.y, (size_t)n * 4));
+    if (clear && other != g_p.bn.x && !overlap((const char*)other, (size_t)n * 4, (const char*)out, (size_t)n * 4)) {
       rd(other, (size_t)n * 4); wr(out, (size_t)n * 4);
       g_p.has_add = true; g_p.add = {a, b, out, n};
       return true;
@@ -406,6 +477,7 @@ bool take_relu_inplace(float* y, int64_t n) {
   }
   if (g_p.kind == P_BN && !g_p.has_add && g_p.bn.y == y && g_p.bn.n == n) {
     Parked p = std::move(g_p); g_p = Parked();
+    if (p.bn.infer) { launch_infer_chain(p, 1, nullptr, y); refresh_busy(); return true; }
     { Replay r_; launch_bn_chain(p, 1, nullptr, y); }
     g_records.push_back({y, p.bn.x, p.bn.beta, n});
     g_stat[ST_FUSED_FWD]++;
@@ -415,6 +487,7 @@ bool take_relu_inplace(float* y, int64_t n) {
   if (g_p.kind == P_BN && g_p.has_add && g_p.add.out == y && g_p.add.n == n) {
     Parked p = std::move(g_p); g_p = Parked();
     const float* other = p.bn.y == p.add.a ? p.add.b : p.add.a;
+    if (p.bn.infer) { launch_infer_chain(p, 1, other, y); refresh_busy(); return true; }
     { Replay r_; launch_bn_chain(p, 1, other, y); }
     // the batch norm's own output was never stored
     Unwritten v{}; v.kind = V_BN_OUT; v.dst = (char*)p.bn.y; v.bytes = (size_t)n * 4; v.n = n;
@@ -517,7 +590,17 @@ bool gather_update(int mode, float* x, float* d, float* v, float lr, float mu, f
 void forget_forward_records() { g_records.clear(); }
 void reset() { g_p = Parked(); g_zero.clear(); g_unwritten.clear(); g_records.clear(); layouts_drop(); g_busy = false; g_replay = false; }
 
+// An inference chain's result that stays, made from what is released, is produced before it goes.
+static void produce_from_released(const char* from) {
+  for (size_t i = 0; i < g_unwritten.size();) {
+    const Unwritten& v = g_unwritten[i];
+    const bool gone = v.kind == V_CONV ? ((const char*)v.conv.x >= from || (const char*)v.conv.w >= from || (const char*)v.conv.bias >= from)
+                                       : v.kind == V_BN_INFER && ((const char*)v.x >= from || (const char*)v.gamma >= from || (const char*)v.beta >= from || (const char*)v.sm >= from || (const char*)v.si >= from);
+    if (gone && v.dst < from) { const Unwritten copy = v; g_unwritten.erase(g_unwritten.begin() + i); produce(copy); i = 0; } else i++;
+  }
+}
 void arena_released(char* from) {
+  if (!g_unwritten.empty()) produce_from_released(from);
   if (!g_layouts.empty()) layouts_released(from);
   while (!g_zero.empty() && g_zero.back().p >= from) g_zero.pop_back();
   for (size_t i = 0; i < g_unwritten.size();) {
@@ -542,7 +625,7 @@ void on_rewind(char* new_top) {
   for (size_t i = 0; i < g_unwritten.size();) {
     const Unwritten& v = g_unwritten[i];
     const bool dangling = v.kind == V_MASK ? ((const char*)v.src >= new_top || (const char*)v.y >= new_top)
-                                           : ((const char*)v.x >= new_top || (const char*)v.sm >= new_top || (const char*)v.si >= new_top);
+                                           : v.kind == V_BN_OUT && ((const char*)v.x >= new_top || (const char*)v.sm >= new_top || (const char*)v.si >= new_top);
     if (dangling) { const Unwritten copy = v; g_unwritten.erase(g_unwritten.begin() + i); produce(copy); i = 0; } else i++;
   }
   refresh_busy();
