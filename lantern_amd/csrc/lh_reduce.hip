@@ -2,6 +2,7 @@
 // over the middle axis of an [outer, c, inner] view, nllLoss.  Wavefront-shuffle (64 lanes)
 // reductions with one LDS hop across the waves of a block.
 #include "lh_common.h"
+#include <type_traits>
 using namespace lh;
 
 namespace {
@@ -99,22 +100,92 @@ __global__ void __launch_bounds__(TPB) k_sum_dim_grad(float* dx, const float* __
 }
 
 // ---- softmax / logSoftmax --------------------------------------------------------------
-// inner == 1: one block per row when c is large, one wave per row when c <= 1024.
-template <bool LOG>
-__global__ void __launch_bounds__(TPB) k_softmax_rows_wave(const float* __restrict__ x, float* __restrict__ y, int rows, int c) {
-  const int lane = threadIdx.x & 63;
-  int64_t w = ((int64_t)blockIdx.x * TPB + threadIdx.x) >> 6, nw = ((int64_t)gridDim.x * TPB) >> 6;
-  for (; w < rows; w += nw) {
-    const float* xp = x + w * c; float* yp = y + w * c;
-    float mx = -3.402823466e+38f;
-    for (int j = lane; j < c; j += 64) mx = fmaxf(mx, xp[j]);
-    mx = lh_wave_max(mx); mx = __shfl(mx, 0, 64);
-    float sum = 0.f;
-    for (int j = lane; j < c; j += 64) sum += expf(xp[j] - mx);
-    sum = lh_wave_sum(sum); sum = __shfl(sum, 0, 64);
-    if (LOG) { float ls = mx + logf(sum); for (int j = lane; j < c; j += 64) yp[j] = xp[j] - ls; }
-    else { for (int j = lane; j < c; j += 64) yp[j] = expf(xp[j] - mx) / sum; }
+// inner == 1, rows of up to SM_REG * TPB elements: NW wavefronts per row (blocks of 4 / NW rows), the row in registers, read once.
+// 8192x4096 (log) 97 -> 43 us, 64x1000 10.9 -> 3.6 us against one wavefront per row that reads it three times.
+constexpr int SM_REG = 16;
+template <int NW>
+__device__ __forceinline__ float row_sum(float v, float* sm) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  if (NW == 1) return v;
+  __syncthreads();                       // (a second sum of the block: the first one's values have been read)
+  if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return (sm[0] + sm[1]) + (sm[2] + sm[3]);
+}
+template <int NW>
+__device__ __forceinline__ float row_max(float v, float* sm) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
+  if (NW == 1) return v;
+  if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return fmaxf(fmaxf(sm[0], sm[1]), fmaxf(sm[2], sm[3]));
+}
+template <bool LOG, int NW, int E>
+__global__ void __launch_bounds__(TPB) k_softmax_rows(const float* x, float* y, int rows, int c) {
+  __shared__ float sm[4];
+  const int t = threadIdx.x & (64 * NW - 1);
+  const int64_t row = NW == 1 ? (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
+  if (row >= rows) return;               // (a whole wavefront, and only where no barrier follows)
+  const float* xp = x + row * c; float* yp = y + row * c;
+  float v[E];
+#pragma unroll
+  for (int e = 0; e < E; e++) { const int j = t + 64 * NW * e; v[e] = j < c ? xp[j] : -3.402823466e+38f; }
+  float mx = v[0];
+#pragma unroll
+  for (int e = 1; e < E; e++) mx = fmaxf(mx, v[e]);
+  mx = fmaxf(row_max<NW>(mx, sm), -3.402823466e+38f);
+  float ex[LOG ? 1 : E], sum = 0.f;
+#pragma unroll
+  for (int e = 0; e < E; e++) {
+    const float w = t + 64 * NW * e < c ? expf(v[e] - mx) : 0.f;
+    if (!LOG) ex[LOG ? 0 : e] = w;
+    sum += w;
   }
+  sum = row_sum<NW>(sum, sm);
+  const float ls = LOG ? mx + logf(sum) : 0.f;
+#pragma unroll
+  for (int e = 0; e < E; e++) { const int j = t + 64 * NW * e; if (j < c) yp[j] = LOG ? v[e] - ls : ex[LOG ? 0 : e] / sum; }
+}
+// Gradient over the same rows: log: dx (+)= dy - exp(y) sum(dy); plain: dx (+)= y (dy - sum(dy y)).  FRESH: dx is a zero block nobody has
+// touched, written instead of added to.  8192x4096 (log) 157 -> 86 us (what its three passes over memory cost), 64x1000 13.0 -> 4.2 us.
+template <bool LOG, bool FRESH, int NW, int E>
+__global__ void __launch_bounds__(TPB) k_softmax_rows_grad(const float* y, const float* dy, float* dx, int rows, int c) {
+  __shared__ float sm[4];
+  const int t = threadIdx.x & (64 * NW - 1);
+  const int64_t row = NW == 1 ? (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
+  if (row >= rows) return;
+  const float* yp = y + row * c; const float* gp = dy + row * c; float* xp = dx + row * c;
+  float v[E], g[E], d[FRESH ? 1 : E], acc = 0.f;
+#pragma unroll
+  for (int e = 0; e < E; e++) {
+    const int j = t + 64 * NW * e;
+    v[e] = j < c ? yp[j] : 0.f; g[e] = j < c ? gp[j] : 0.f;
+    if (!FRESH) d[FRESH ? 0 : e] = j < c ? xp[j] : 0.f;
+  }
+#pragma unroll
+  for (int e = 0; e < E; e++) acc += LOG ? g[e] : g[e] * v[e];
+  acc = row_sum<NW>(acc, sm);
+#pragma unroll
+  for (int e = 0; e < E; e++) {
+    const int j = t + 64 * NW * e;
+    const float r = LOG ? g[e] - expf(v[e]) * acc : v[e] * (g[e] - acc);
+    if (j < c) xp[j] = (FRESH ? 0.f : d[FRESH ? 0 : e]) + r;
+  }
+}
+// Wavefronts per row: one for short rows, four where the rows are few (their latency counts) or long.  `go` gets (wavefronts, elements a thread).
+template <class F>
+static bool softmax_plan(int64_t rows, int c, F go) {
+  const bool four = c > 64 * SM_REG || (c > 256 && rows < 8 * (int64_t)g_num_cu);
+  const int per = (int)cdiv(c, four ? TPB : 64);
+  if (per > SM_REG || rows > 0x7fffffff) return false;
+  const unsigned grid = (unsigned)(four ? rows : cdiv(rows, 4));
+  if (four) { if (per <= 4) go(std::integral_constant<int, 4>(), std::integral_constant<int, 4>(), grid); else go(std::integral_constant<int, 4>(), std::integral_constant<int, SM_REG>(), grid); }
+  else if (per <= 1) go(std::integral_constant<int, 1>(), std::integral_constant<int, 1>(), grid);
+  else if (per <= 4) go(std::integral_constant<int, 1>(), std::integral_constant<int, 4>(), grid);
+  else go(std::integral_constant<int, 1>(), std::integral_constant<int, SM_REG>(), grid);
+  return true;
 }
 template <bool LOG>
 __global__ void __launch_bounds__(TPB) k_softmax_rows_block(const float* __restrict__ x, float* __restrict__ y, int c) {
@@ -211,11 +282,11 @@ void lh_softmax(int is_log, const float* x, float* y, int outer, int c, int inne
   if ((int64_t)outer * c * inner <= 0) return;
   if (inner == 1 && rec_ok((int64_t)outer * c)) { rec_cmd(CL_SOFTMAX, outer, c, is_log ? 1 : 0, 0.f, 0.f, 0.f, 0.f, y, x, nullptr, nullptr); return; }
   if (inner == 1) {
-    if (c <= 1024 || outer >= 4 * g_num_cu) {
-      int grid = stream_grid((int64_t)outer * 64, TPB);
-      if (is_log) hipLaunchKernelGGL((k_softmax_rows_wave<true>), dim3(grid), dim3(TPB), 0, g_stream, x, y, outer, c);
-      else hipLaunchKernelGGL((k_softmax_rows_wave<false>), dim3(grid), dim3(TPB), 0, g_stream, x, y, outer, c);
-    } else {
+    const bool done = softmax_plan(outer, c, [&](auto NW, auto E, unsigned grid) {
+      if (is_log) hipLaunchKernelGGL((k_softmax_rows<true, decltype(NW)::value, decltype(E)::value>), dim3(grid), dim3(TPB), 0, g_stream, x, y, outer, c);
+      else hipLaunchKernelGGL((k_softmax_rows<false, decltype(NW)::value, decltype(E)::value>), dim3(grid), dim3(TPB), 0, g_stream, x, y, outer, c);
+    });
+    if (!done) {
       if (is_log) hipLaunchKernelGGL((k_softmax_rows_block<true>), dim3(outer), dim3(TPB), 0, g_stream, x, y, c);
       else hipLaunchKernelGGL((k_softmax_rows_block<false>), dim3(outer), dim3(TPB), 0, g_stream, x, y, c);
     }
@@ -226,10 +297,21 @@ void lh_softmax(int is_log, const float* x, float* y, int outer, int c, int inne
   }
   LH_CHECK_LAUNCH();
 }
-void lh_softmax_grad(int is_log, const float* y, const float* dy, float* dx, int outer, int c, int inner) { LZ_ENTER(); lazy::rd_f(y, (int64_t)outer * c * inner); lazy::rd_f(dy, (int64_t)outer * c * inner); lazy::rw_f(dx, (int64_t)outer * c * inner); ProfScope prof_(CAT_REDUCE);
+void lh_softmax_grad(int is_log, const float* y, const float* dy, float* dx, int outer, int c, int inner) { LZ_ENTER(); lazy::rd_f(y, (int64_t)outer * c * inner); lazy::rd_f(dy, (int64_t)outer * c * inner);
   int64_t groups = (int64_t)outer * inner;
+  const bool in_registers = inner == 1 && c <= SM_REG * TPB && !rec_ok(groups * c);
+  bool fresh = false;
+  if (in_registers) fresh = lazy::acc_f(dx, groups * c); else lazy::rw_f(dx, groups * c);
+  ProfScope prof_(CAT_REDUCE);
   if (groups * c <= 0) return;
   if (inner == 1 && rec_ok(groups * c)) { rec_cmd(CL_SOFTMAX_GRAD, outer, c, is_log ? 1 : 0, 0.f, 0.f, 0.f, 0.f, dx, y, dy, nullptr); return; }
+  if (in_registers && softmax_plan(groups, c, [&](auto NW, auto E, unsigned grid) {
+        constexpr int W = decltype(NW)::value, N = decltype(E)::value;
+        if (is_log) { if (fresh) hipLaunchKernelGGL((k_softmax_rows_grad<true, true, W, N>), dim3(grid), dim3(TPB), 0, g_stream, y, dy, dx, outer, c);
+                      else hipLaunchKernelGGL((k_softmax_rows_grad<true, false, W, N>), dim3(grid), dim3(TPB), 0, g_stream, y, dy, dx, outer, c); }
+        else { if (fresh) hipLaunchKernelGGL((k_softmax_rows_grad<false, true, W, N>), dim3(grid), dim3(TPB), 0, g_stream, y, dy, dx, outer, c);
+               else hipLaunchKernelGGL((k_softmax_rows_grad<false, false, W, N>), dim3(grid), dim3(TPB), 0, g_stream, y, dy, dx, outer, c); }
+      })) { LH_CHECK_LAUNCH(); return; }
   int grid = stream_grid(groups * 64, TPB);
   if (is_log) hipLaunchKernelGGL((k_softmax_grad_wave<true>), dim3(grid), dim3(TPB), 0, g_stream, y, dy, dx, groups, c, inner);
   else hipLaunchKernelGGL((k_softmax_grad_wave<false>), dim3(grid), dim3(TPB), 0, g_stream, y, dy, dx, groups, c, inner);
