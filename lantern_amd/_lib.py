@@ -6,6 +6,11 @@ if the shared object is missing or a symbol does not resolve, loading raises.
 import ctypes as C
 import os
 
+try:
+    from . import _lhpy          # csrc/lh_py.cpp: calls, handles and checks without ctypes (built beside the library)
+except ImportError:              # another interpreter than the one it was built for: ctypes does the same, slower
+    _lhpy = None
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "csrc", "liblantern_hip.so")
 
@@ -140,6 +145,10 @@ SIGNATURES = {
     "lh_multi_momentum_static": (None, [I, P, P, P, P, F, F, F, I]),
 }
 
+# Entry points called once, or that wait for the device: a few microseconds of ctypes don't show there.
+WAITS = {"lh_setup", "lh_cleanup", "lh_sync", "lh_h2d", "lh_d2h", "lh_clear_error", "lh_flush_deferred", "lh_side_join", "lh_copy_join", "lh_cmdlist_begin",
+         "lh_cmdlist_end", "lh_capture_begin"}
+
 _lib = None
 
 
@@ -168,6 +177,14 @@ def load():
     _err_flag = C.c_ubyte.from_address(lib.lh_last_error())
     lib.lh_last_error.restype = C.c_char_p
     _lib = lib
+    if _lhpy is not None:
+        global check
+        check = _lhpy.check(C.addressof(_err_flag), check)
+        letters = {None: "v", P: "P", I: "I", F: "F", L: "L", Z: "Z"}
+        for name, (res, args) in SIGNATURES.items():
+            if res in letters and name not in WAITS and all(a in letters for a in args):
+                fn = getattr(lib, name)
+                setattr(lib, name, _lhpy.call(letters[res] + "".join(letters[a] for a in args), C.cast(fn, P).value, fn))
     return lib
 
 

@@ -19,7 +19,7 @@ ADD, SUB, MUL, DIV = 0, 1, 2, 3
 RELU, TANH, SIGMOID, EXP, LOG, SQRT, SQUARE, HARDTANH = range(8)
 
 
-class Buf:
+class PyBuf:
     """A span of backend memory: address, element count (4-byte elements) and an owner to keep alive."""
     __slots__ = ("ptr", "n", "keep")
 
@@ -31,6 +31,9 @@ class Buf:
     def offset(self, k, n=None):
         """`slice(arr, off)` of the reference (TD:55): same memory, starting k elements in."""
         return Buf(self.ptr + 4 * int(k), self.n - int(k) if n is None else n, self.keep)
+
+
+Buf = PyBuf if _lib._lhpy is None else _lib._lhpy.Buf          # the same, without an entry in the garbage collector
 
 
 _INTS_CACHE = {}
@@ -49,6 +52,8 @@ def _ints(seq):
 
 def dim_broadcast(a, b):
     """Tensor.dimBroadcast (TD:997-1016): right-aligned numpy rules -> (aShape, bShape, resShape)."""
+    if a == b and type(a) is tuple and type(b) is tuple:
+        return a, b, a
     a, b = list(a), list(b)
     r = max(len(a), len(b))
     a = [1] * (r - len(a)) + a
@@ -356,7 +361,9 @@ class BackendHIP(Backend):
 
     # -- broadcast arithmetic (TD:222-270) ---------------------------------------------------------
     def bcast_op(self, op, a, ashape, b, bshape, oshape):
-        n = int(np.prod(oshape, dtype=np.int64))
+        n = 1
+        for d in oshape:
+            n *= int(d)
         res = self.mallocArray(n)
         self.lib.lh_bcast_op(op, a.ptr, _ints(ashape), b.ptr, _ints(bshape), res.ptr, _ints(oshape), len(oshape)); _lib.check()
         return res

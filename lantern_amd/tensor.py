@@ -72,6 +72,7 @@ class Random:
 
 class Tensor:
     """Dense row-major fp32 tensor: a backend buffer plus dims (TD:386-398)."""
+    __slots__ = ("data", "shape", "scalarCount", "rank", "__dict__", "__weakref__")      # (a dictionary only for what a program adds)
 
     def __init__(self, data, dims):
         self.data = data
@@ -113,7 +114,7 @@ class Tensor:
 
     @staticmethod
     def zeros_like(t):
-        return Tensor(get_backend().mallocArray(t.scalarCount), t.shape)
+        return _like(get_backend().mallocArray(t.scalarCount), t)
 
     @staticmethod
     def fill(dims, value):
@@ -258,7 +259,7 @@ class Tensor:
 
     # -- activations -------------------------------------------------------------------------------
     def _unary(self, op, inPlace=False, lo=-1.0, hi=1.0):
-        return Tensor(get_backend().unary(op, self.data, self.scalarCount, inPlace, lo, hi), self.shape)
+        return _like(get_backend().unary(op, self.data, self.scalarCount, inPlace, lo, hi), self)
 
     def relu(self, inPlace=False): return self._unary(B.RELU, inPlace)
     def tanh(self): return self._unary(B.TANH)
@@ -406,8 +407,56 @@ def int_array(values):
     return get_backend().fromHost(np.asarray(values, dtype=np.int32))
 
 
+def _like(data, t):
+    """A Tensor of t's shape over `data`."""
+    r = Tensor.__new__(Tensor)
+    r.data, r.shape, r.scalarCount, r.rank = data, t.shape, t.scalarCount, t.rank
+    return r
+
+
+# A tape entry is a callable, or a tuple of one and its arguments: one object for the garbage collector instead of a function, its
+# closure and a cell per variable.  Buffers are looked up when the entry runs, so an entry holds the TensorRs.
+def _accumulate(to, y):
+    if not to.isInput:
+        to.d += y.d
+
+
+def _bin_back(be, op, x, a, that, b, y):
+    be.bcast_op_grad(op, x.x.data, x.d.data, a, x.isInput, that.x.data, that.d.data, b, that.isInput, y.d.data, y.x.shape)
+
+
+def _unary_back(be, op, x, y, inPlace, lo, hi):
+    be.unary_grad(op, x.x.data, y.x.data, y.d.data, x.d.data, x.x.scalarCount, inPlace, lo, hi)
+
+
+def _dot_back(be, x, that, y):                                                        # dot_grad (CPU:171-184)
+    xr, yr = x.x.rank, that.x.rank
+    if xr == 1 and yr == 1:
+        if not x.isInput: be.addMul_scalar(x.d.data, y.d.data, that.x.data, x.x.scalarCount)
+        if not that.isInput: be.addMul_scalar(that.d.data, y.d.data, x.x.data, that.x.scalarCount)
+    elif xr == 2 and yr == 1:
+        m, n = x.x.shape
+        if not x.isInput: be.add_cartesian(x.d.data, that.x.data, y.d.data, m, n)
+        if not that.isInput: be.add_composition(that.d.data, x.x.data, y.d.data, m, n)
+    else:
+        d1, d2 = x.x.shape; d3 = that.x.shape[1]
+        if not x.isInput: be.add_dotTrans2(x.d.data, y.d.data, that.x.data, d1, d2, d3)
+        if not that.isInput: be.add_dotTrans1(that.d.data, x.x.data, y.d.data, d1, d2, d3)
+
+
+def _conv_back(be, x, kernel, bias, finput, y, geom):
+    be.convs_open -= 1
+    be.conv2D_batch_grad(x.x.data, None if x.isInput else x.d.data, x.isInput, finput, kernel.x.data, kernel.d.data, y.d.data,
+                         bias.d.data if bias is not None else None, *geom)
+
+
+def _batchNorm_back(be, x, y, scale, bias, sm, si, geom):
+    be.batchNorm_grad(x.x.data, None if x.isInput else x.d.data, y.d.data, scale.x.data, scale.d.data, bias.d.data, sm.data, si.data, *geom)
+
+
 class TensorR:
     """A value with its gradient (TD:1146-1506).  `d` accumulates; inputs never receive one."""
+    __slots__ = ("x", "d", "isInput", "__dict__", "__weakref__")
 
     def __init__(self, x, d=None, isInput=False):
         """The gradient is allocated zero-filled at construction; an input gets a 2-element dummy (TD:1509-1514)."""
@@ -432,18 +481,12 @@ class TensorR:
     # -- in-place adds --------------------------------------------------------------------------
     def plusBias(self, bias):
         self.x.plusBias(bias.x)
-        def back():
-            if not bias.isInput:
-                bias.d += self.d                 # reduce main.d into bias.d (CPU:286-288)
-        _tape.append(back)
+        _tape.append((_accumulate, bias, self))      # reduce main.d into bias.d (CPU:286-288)
         return self
 
     def plusEqual(self, that):
         self.x.plusEqual(that.x)
-        def back():
-            if not that.isInput:
-                that.d += self.d
-        _tape.append(back)
+        _tape.append((_accumulate, that, self))
         return self
 
     # -- arithmetic --------------------------------------------------------------------------------
@@ -453,7 +496,7 @@ class TensorR:
             ya, a, b = self.x._bin(op, that.x)
             y = TensorR._new(ya)
             # add_grad / minus_grad / mul_grad / div_grad (TD:1171-1206): both operands' gradients in one backend call
-            _tape.append(lambda: be.bcast_op_grad(op, self.x.data, self.d.data, a, self.isInput, that.x.data, that.d.data, b, that.isInput, y.d.data, ya.shape))
+            _tape.append((_bin_back, be, op, self, a, that, b, y))
             return y
         s = float(that)
         y = TensorR._new(self.x._bin(op, s))
@@ -473,20 +516,7 @@ class TensorR:
     def dot(self, that):
         be = get_backend()
         y = TensorR._new(self.x.dot(that.x))
-        def back():                                                                   # dot_grad (CPU:171-184)
-            xr, yr = self.x.rank, that.x.rank
-            if xr == 1 and yr == 1:
-                if not self.isInput: be.addMul_scalar(self.d.data, y.d.data, that.x.data, self.x.scalarCount)
-                if not that.isInput: be.addMul_scalar(that.d.data, y.d.data, self.x.data, that.x.scalarCount)
-            elif xr == 2 and yr == 1:
-                m, n = self.x.shape
-                if not self.isInput: be.add_cartesian(self.d.data, that.x.data, y.d.data, m, n)
-                if not that.isInput: be.add_composition(that.d.data, self.x.data, y.d.data, m, n)
-            else:
-                d1, d2 = self.x.shape; d3 = that.x.shape[1]
-                if not self.isInput: be.add_dotTrans2(self.d.data, y.d.data, that.x.data, d1, d2, d3)
-                if not that.isInput: be.add_dotTrans1(that.d.data, self.x.data, y.d.data, d1, d2, d3)
-        _tape.append(back)
+        _tape.append((_dot_back, be, self, that, y))
         return y
 
     def gemm(self, that, transX, transY, alpha):
@@ -511,10 +541,10 @@ class TensorR:
         be = get_backend()
         if inPlace:
             self.x._unary(op, True, lo, hi)
-            _tape.append(lambda: be.unary_grad(op, self.x.data, self.x.data, self.d.data, self.d.data, self.x.scalarCount, True, lo, hi))
+            _tape.append((_unary_back, be, op, self, self, True, lo, hi))
             return self
         y = TensorR._new(self.x._unary(op, False, lo, hi))
-        _tape.append(lambda: be.unary_grad(op, self.x.data, y.x.data, y.d.data, self.d.data, self.x.scalarCount, False, lo, hi))
+        _tape.append((_unary_back, be, op, self, y, False, lo, hi))
         return y
 
     def relu(self, inPlace=False): return self._unary(B.RELU, inPlace)
@@ -556,8 +586,7 @@ class TensorR:
         N, C, HW = self.x._bn_view()
         yv, sm, si = self.x.batchNormTraining(scale.x, bias.x, runningMean, runningVar)
         y = TensorR._new(yv)
-        _tape.append(lambda: be.batchNorm_grad(self.x.data, None if self.isInput else self.d.data, y.d.data, scale.x.data, scale.d.data, bias.d.data,
-                                               sm.data, si.data, N, C, HW))
+        _tape.append((_batchNorm_back, be, self, y, scale, bias, sm, si, (N, C, HW)))
         return y
 
     batchNorm1D = batchNorm
@@ -594,11 +623,7 @@ class TensorR:
         yv, finput = self.x.conv2D_batch(kernel.x, bias.x if bias is not None else None, strides, pads)
         y = TensorR._new(yv)
         be.convs_open += 1                  # forward convolutions whose gradient is still to come (a backend may run filter gradients beside the ones that follow)
-        def back():
-            be.convs_open -= 1
-            be.conv2D_batch_grad(self.x.data, None if self.isInput else self.d.data, self.isInput, finput, kernel.x.data, kernel.d.data, y.d.data,
-                                 bias.d.data if bias is not None else None, N, C, H, W, K, R, S, sH, sW, pH, pW)
-        _tape.append(back)
+        _tape.append((_conv_back, be, self, kernel, bias, finput, y, (N, C, H, W, K, R, S, sH, sW, pH, pW)))
         return y
 
     def maxPoolBK(self, kernels, strides, pads=None):
@@ -693,7 +718,9 @@ class TensorR:
 
 def _run_tape(start):
     while len(_tape) > start:
-        _tape.pop()()
+        entry = _tape.pop()
+        if type(entry) is tuple: entry[0](*entry[1:])
+        else: entry()
 
 
 def gradR(f):
