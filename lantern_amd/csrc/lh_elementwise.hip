@@ -446,7 +446,7 @@ static bool col_sums(float* small, const float* big, int rows, int cols, float s
   const size_t bytes = slices > 1 ? (size_t)slices * cols * sizeof(float) : 0;
   float* partial = nullptr;
   if (bytes) {
-    if (g_stream_cur == g_stream_raw && arena_room() < bytes + 256) return false;
+    if (g_capturing || (g_stream_cur == g_stream_raw && arena_room() < bytes + 256)) return false;      // (a replay would write to arena memory that may have been handed out since)
     partial = (float*)scratch_take(bytes, side);
     if (partial == nullptr) return true;                  // (reported)
   }

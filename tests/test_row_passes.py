@@ -101,3 +101,25 @@ def test_broadcast_over_rows(on_hip, full, small, op):
         assert (np.abs(d.down(gb, small) - (b + s64 if op == B.ADD else b - s64)) <= tol).all()
         np.testing.assert_array_equal(d.down(ga, full), a)
     on_hip.resetMallocAddr(mark)
+
+
+def test_recorded_column_sums_leave_memory_handed_out_later_alone(on_hip):
+    """A graph's replay runs what was recorded at the addresses it was recorded with: partial sums kept above the arena's top would land
+    in what the program has allocated there since."""
+    d, rows, cols = Dev(on_hip), 4096, 96
+    mark = on_hip.getMallocAddr()
+    a = np.random.RandomState(3).standard_normal((rows, cols)).astype(np.float32)
+    A, t = d.up(a), d.zeros(cols)
+    on_hip.toHost(t, cols)
+    on_hip.captureBegin()
+    on_hip.lib.lh_bcast_update(B.ADD, t.ptr, B._ints((1, cols)), A.ptr, B._ints((rows, cols)), 2); _lib.check()
+    graph = on_hip.captureEnd()
+    later = np.arange(1 << 16, dtype=np.float32)
+    held = d.up(later)
+    for r in range(1, 4):
+        on_hip.graphLaunch(graph)
+        tol = r * (np.sqrt(rows) + 8) * 2.0 ** -24 * np.sqrt(rows * 16.0)
+        assert (np.abs(d.down(t, (cols,)) - r * a.astype(np.float64).sum(0)) <= tol).all()
+        np.testing.assert_array_equal(d.down(held, (1 << 16,)), later)
+    on_hip.graphDestroy(graph)
+    on_hip.resetMallocAddr(mark)
