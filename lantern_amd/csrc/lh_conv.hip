@@ -424,7 +424,12 @@ static bool launch_rounds(const AL& al, const BL& bl, const EP& ep, int M, int N
 // as large as the map: a fully connected layer), where a worker per CU would mean hundreds of atomic adds onto each element.
 // 13-15: whole 64x64 / 64x128 / 128x128 tiles, the last ones (what is left over a multiple of the compute units) cut into
 // slices along the reduction and finished by whichever slice arrives last (igemm_launch_shared_tail).
-constexpr int N_PLANS = 16;
+// 16-18: 64x64 tiles on blocks of two or four groups of wavefronts that share a tile's slabs (igemm_block): whole tiles on two and on
+// four, plan 13 on two; for launches of a few tiles per compute unit (beyond eight none of them was ever the fastest of a ResNet-50's
+// shapes) with at least four slabs a group.  Steps with them and without, one card in turn: ResNet-50 on 32x32 images 3.61 | 3.79 ms,
+// batch 21 at 161x161 6.27 | 6.39, batch 64 at 224x224 17.70 | 17.86, DeepSpeech 8.49 | 8.60.
+constexpr int N_PLANS = 19;
+static inline bool deep_ok(int M, int N, int K, int groups) { return !g_deterministic && cdiv(K, CONV_BK) >= 4 * groups && cdiv(M, 64) * cdiv(N, 64) <= 8 * (int64_t)g_num_cu; }
 // LH_FORCE_M32 in the environment: products of at most 32 rows always take the 32-row tile (for tests of that tile; the
 // measured choice may well be another one).
 static inline bool force_m32() { return getenv("LH_FORCE_M32") != nullptr; }
@@ -435,7 +440,8 @@ static inline bool no_split_gather() { const char* e = getenv("LH_NO_SPLIT_GATHE
 // LH_FORCE_STATS_TILE=f: the same for the forward launches that leave batch-norm statistics behind (f as in conv_fwd_impl's `run`).
 static inline int force_stats_tile() { const char* e = getenv("LH_FORCE_STATS_TILE"); return e ? atoi(e) : -1; }
 template <class AL, class BL, class EP>
-static bool plan_valid(int plan, const EP& ep, int M, int K, bool can_zero) {
+static bool plan_valid(int plan, const EP& ep, int M, int N, int K, bool can_zero) {
+  if (plan >= 16) return deep_ok(M, N, K, plan == 17 ? 4 : 2) && (plan != 18 || g_stream_cur == g_stream_raw);
   if (plan == 0) return true;
   if (plan == 10) return M <= 32;
   if ((plan == 1 || plan == 4 || plan == 6) && M <= 64) return false;
@@ -454,6 +460,9 @@ static bool launch_plan(int plan, const AL& al, const BL& bl, const EP& ep, int 
   if (plan == 13) return igemm_launch_shared_tail<64, 64, CONV_BK>(al, bl, ep, M, N, K);
   if (plan == 14) return igemm_launch_shared_tail<64, 128, CONV_BK>(al, bl, ep, M, N, K);
   if (plan == 15) return igemm_launch_shared_tail<128, 128, CONV_BK>(al, bl, ep, M, N, K);
+  if (plan == 16) return igemm_launch_shared_tail<64, 64, CONV_BK, 2>(al, bl, ep, M, N, K, 1);
+  if (plan == 17) return igemm_launch_shared_tail<64, 64, CONV_BK, 4>(al, bl, ep, M, N, K, 1);
+  if (plan == 18) return igemm_launch_shared_tail<64, 64, CONV_BK, 2>(al, bl, ep, M, N, K);
   if (plan >= 11) {
     g_launch_partial = true;
     const int64_t units = cdiv(M, 64) * cdiv(N, 64) * cdiv(K, CONV_BK);
@@ -499,7 +508,7 @@ static bool launch_tiles(const AL& al, const BL& bl, const EP& ep, int M, int N,
   const bool can_zero = zero_out != nullptr || prezeroed;
   if (M <= 32 && force_m32()) return launch_plan(10, al, bl, ep, M, N, K, zero_out, zero_n, prezeroed);
   const int forced = force_plan();
-  if (forced >= 0 && forced < N_PLANS && plan_valid<AL, BL, EP>(forced, ep, M, K, can_zero)) return launch_plan(forced, al, bl, ep, M, N, K, zero_out, zero_n, prezeroed);
+  if (forced >= 0 && forced < N_PLANS && plan_valid<AL, BL, EP>(forced, ep, M, N, K, can_zero)) return launch_plan(forced, al, bl, ep, M, N, K, zero_out, zero_n, prezeroed);
   // Deterministic mode keeps the measured choice among the plans whose tiles are finished by one block each: they add the same
   // terms in the same order whatever the tile shape, so which of them runs changes no bit (tests/test_parity_conv.py compares them).
   if (!g_tune_enabled || 2.0 * M * N * (double)K < g_tune_min_flop) return launch_plan(0, al, bl, ep, M, N, K, zero_out, zero_n, prezeroed);
@@ -507,40 +516,43 @@ static bool launch_tiles(const AL& al, const BL& bl, const EP& ep, int M, int N,
   auto it = chosen.find(key);
   if (it != chosen.end()) {
     g_plans_remembered++;
-    const int plan = plan_valid<AL, BL, EP>(it->second, ep, M, K, can_zero) ? it->second : 0;
+    const int plan = plan_valid<AL, BL, EP>(it->second, ep, M, N, K, can_zero) ? it->second : 0;
     return launch_plan(plan, al, bl, ep, M, N, K, zero_out, zero_n, prezeroed);
   }
   // tuned only on a call that may be repeated: an overwriting epilogue onto an output this launch alone writes
   if (g_capturing || ep.beta != 0.f || prezeroed) return launch_plan(0, al, bl, ep, M, N, K, zero_out, zero_n, prezeroed);
   LaunchTimer timer;
   if (!timer.ok) return launch_plan(0, al, bl, ep, M, N, K, zero_out, zero_n, prezeroed);
-  int best = 0; float best_ms = 3.0e38f, base_ms = 0.f;
+  int best = 0, last = 0; float best_ms = 3.0e38f, base_ms = 0.f;
   for (int plan = 0; plan < N_PLANS; plan++) {
-    if (!plan_valid<AL, BL, EP>(plan, ep, M, K, can_zero)) continue;
+    if (!plan_valid<AL, BL, EP>(plan, ep, M, N, K, can_zero)) continue;
     const float ms = timer.ms([&]() { return launch_plan(plan, al, bl, ep, M, N, K, zero_out, zero_n, prezeroed); });
     if (ms < 0.f || failed()) return false;
     if (plan == 0) base_ms = ms;
+    last = plan;
     if (ms < best_ms * 0.98f) { best_ms = ms; best = plan; }      // a later plan must win by 2 % to displace an earlier one
   }
   chosen[key] = best; g_plans_measured++;
   if (getenv("LH_TUNE_VERBOSE")) fprintf(stderr, "conv product M%d N%d K%d (stride %d,%d): plan %d, %.3f ms (built-in rule %.3f ms)\n", M, N, K, ep.eH, ep.eW, best, best_ms, base_ms);
-  return true;                                               // the timed launches have produced the result
+  // (the plans do not all add in the same order: the first call gives the bits of those that follow)
+  return last == best || launch_plan(best, al, bl, ep, M, N, K, zero_out, zero_n, prezeroed);
 }
 
 // Where the statistics pieces of a forward launch lie (see bn_finalize_conv_partials).
-struct StatLayout { int col1, g_main, slots_main, g_rem, slots_rem; int sliced = 0; };      // sliced: whole tiles and slices of the last ones (igemm_launch_shared_tail)
+struct StatLayout { int col1, g_main, slots_main, g_rem, slots_rem; int sliced = 0, groups = 1; };      // sliced: whole tiles and slices of the last ones (igemm_launch_shared_tail); groups: of wavefronts per block
 
 // The tile plan launch_tiles would choose, for a launch that also leaves statistics pieces.  Returns false (and
 // launches nothing) for shapes that take the stream-K path, whose tiles are finished by several blocks.
 template <class AL, class BL>
-static bool plan_tiles_stats(int M, int N, int K, StatLayout& L, int& bm, int& bn, int force = 0 /* 1-3: the tile of launch plan 1-3; 5-7: 64x64 / 64x128 / 128x128 tiles with the last ones sliced */) {
+static bool plan_tiles_stats(int M, int N, int K, StatLayout& L, int& bm, int& bn, int force = 0 /* 1-3: the tile of launch plan 1-3; 5-7: 64x64 / 64x128 / 128x128 tiles with the last ones sliced; 8-10: launch plans 16-18 */) {
   const int64_t t128 = cdiv(M, 128) * cdiv(N, 128), t64 = cdiv(M, 64) * cdiv(N, 128);
   const bool few = (M > 64 ? t128 : t64) < 6 * (int64_t)g_num_cu;
   const int64_t slabs = cdiv(K, CONV_BK);
   if (!g_deterministic && few && slabs >= 64 && slabs * (M > 64 ? t128 : t64) >= 48 * (int64_t)(2 * g_num_cu)) return false;
   TilePick tp = pick_tile_conv(M, N, K);
-  if ((force == 1 || force == 7) && M > 64) tp = {128, 128}; else if (force == 2 || force == 6) tp = {64, 128}; else if (force == 3 || force == 5) tp = {64, 64};
-  L.sliced = (force == 5 || force == 6 || (force == 7 && M > 64)) && !g_deterministic && g_stream_cur == g_stream_raw && cdiv(K, CONV_BK) >= 8;
+  if ((force == 1 || force == 7) && M > 64) tp = {128, 128}; else if (force == 2 || force == 6) tp = {64, 128}; else if (force == 3 || force == 5 || force >= 8) tp = {64, 64};
+  L.groups = force >= 8 && deep_ok(M, N, K, force == 9 ? 4 : 2) ? (force == 9 ? 4 : 2) : 1;
+  L.sliced = (force == 5 || force == 10 || force == 6 || (force == 7 && M > 64)) && !g_deterministic && g_stream_cur == g_stream_raw && cdiv(K, CONV_BK) >= 8;
   bm = tp.bm; bn = tp.bn;
   L.col1 = N; L.g_main = bn / 2; L.g_rem = 32; L.slots_rem = 0;
   if (bn == 128 && !L.sliced) {        // the surplus-tile split of launch_rounds
@@ -561,6 +573,8 @@ template <class AL, class BL>
 static bool launch_tiles_stats(const AL& al, const BL& bl, EpiConvOutStats ep, int M, int N, int K, const StatLayout& L, int bm, int bn) {
   ep.slotBase = 0;
   bool ok;
+  if (L.groups == 4) return igemm_launch_shared_tail<64, 64, CONV_BK, 4>(al, bl, ep, M, N, K, 1);
+  if (L.groups == 2) return igemm_launch_shared_tail<64, 64, CONV_BK, 2>(al, bl, ep, M, N, K, L.sliced ? 8 : 1);
   if (L.sliced) return bm == 128 ? igemm_launch_shared_tail<128, 128, CONV_BK>(al, bl, ep, M, N, K) : (bn == 128 ? igemm_launch_shared_tail<64, 128, CONV_BK>(al, bl, ep, M, N, K) : igemm_launch_shared_tail<64, 64, CONV_BK>(al, bl, ep, M, N, K));
   if (bm == 128) ok = igemm_launch<128, 128, CONV_BK>(al, bl, ep, M, N, K, 1, 0, 0, L.col1);
   else if (bn == 128) ok = igemm_launch<64, 128, CONV_BK>(al, bl, ep, M, N, K, 1, 0, 0, L.col1);
@@ -610,7 +624,7 @@ static void conv_fwd_impl(const float* x, const float* w, const float* bias, flo
       const PlanKey key = {{K, N * PQ, CRS, H, W, sH, R}};
       const bool tunable = g_tune_lookup && 2.0 * K * CRS * (double)N * PQ >= g_tune_min_flop;
       int force = 0;
-      auto run = [&](int f) {           // 0: the rule's tile, 1-3: a forced tile, 4: unfused (any launch plan, then a pass over y), 5-7: 64x64 / 64x128 / 128x128 tiles, the last ones sliced
+      auto run = [&](int f) {           // 0: the rule's tile, 1-3: a forced tile, 4: unfused (any launch plan, then a pass over y), 5-7: 64x64 / 64x128 / 128x128 tiles, the last ones sliced, 8-10: launch plans 16-18
         if (f == 4) {
           if (!launch_tiles(al, bl, ep, K, N * PQ, CRS, y, (int64_t)N * K * PQ)) return false;
           lh_bn_stats(y, bn->save_mean, bn->save_invstd, nullptr, nullptr, N, K, PQ, bn->eps, bn->factor);
@@ -635,9 +649,10 @@ static void conv_fwd_impl(const float* x, const float* w, const float* bias, flo
           LaunchTimer timer;
           if (timer.ok) {
             float best_ms = 3.0e38f, base_ms = 0.f; int best = 0;
-            for (int f = 0; f <= 7; f++) {
+            for (int f = 0; f <= 10; f++) {
+              if (f >= 8 && !deep_ok(K, N * PQ, CRS, f == 9 ? 4 : 2)) continue;
               if ((f == 1 || f == 7) && K <= 64) continue;
-              if (f >= 5 && (g_deterministic || CRS < 8 * CONV_BK)) continue;
+              if (f >= 5 && f != 8 && f != 9 && (g_deterministic || CRS < 8 * CONV_BK)) continue;
               const float ms = timer.ms([&]() { return run(f); });
               if (ms < 0.f || failed()) return;
               if (f == 0) base_ms = ms;

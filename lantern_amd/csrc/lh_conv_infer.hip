@@ -12,10 +12,16 @@ struct EpiConvBn : EpiConvOut {
   static constexpr bool ROWS = true;
   const float* gamma; const float* shift; const float* mean; const float* var; float eps;
   const float* shortcut;
-  __device__ __forceinline__ float4 row_params(int row, int M) const {
-    if (row >= M) return make_float4(0.f, 0.f, 0.f, 0.f);
-    return make_float4(mean[row], gamma[row] / sqrtf(var[row] + eps), shift[row], bias ? bias[row] : 0.f);
+  // a row's values as they lie in memory (0 past the last row), and what the epilogue makes of them
+  __device__ __forceinline__ float row_load(const float* p, int row, int M) const {
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, M * 4, LH_RSRC_FLAGS);
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, row * 4, 0, 0));
   }
+  __device__ __forceinline__ void row_fetch(int row, int M, float4& v, float& b) const {
+    v = make_float4(row_load(mean, row, M), row_load(gamma, row, M), row_load(shift, row, M), row_load(var, row, M));
+    if (bias) b = row_load(bias, row, M);
+  }
+  __device__ __forceinline__ float4 row_params(const float4 v, float b) const { return make_float4(v.x, v.y / sqrtf(v.w + eps), v.z, b); }
   __device__ __forceinline__ float row_value(float v, const float4 p, float other, bool join) const {
     if (bias) v += p.w;
     float r = fmaf(v - p.x, p.y, p.z);
@@ -33,12 +39,17 @@ struct EpiConvBn : EpiConvOut {
 };
 
 // Launch forms: 1-3 whole tiles 128x128, 64x128, 64x64; 5-7 the last tiles of 64x64 / 64x128 / 128x128 sliced along the reduction
-// (igemm_launch_shared_tail); 4 the convolution by itself (any of its launch plans, stream-K among them), then the pass over it.
+// (igemm_launch_shared_tail); 8-11 64x64 tiles on blocks of two groups of wavefronts, whole and sliced, and of four, whole and sliced;
+// 4 the convolution by itself (any of its launch plans, stream-K among them), then the pass over it.
 template <class AL, class BL>
 bool launch_form(int form, const AL& al, const BL& bl, const EpiConvBn& ep, int M, int N, int K) {
   if (form == 1) return igemm_launch<128, 128, CONV_BK>(al, bl, ep, M, N, K, 1);
   if (form == 2) return igemm_launch<64, 128, CONV_BK>(al, bl, ep, M, N, K, 1);
   if (form == 5) return igemm_launch_shared_tail<64, 64, CONV_BK>(al, bl, ep, M, N, K);
+  if (form == 8) return igemm_launch_shared_tail<64, 64, CONV_BK, 2>(al, bl, ep, M, N, K, 1);
+  if (form == 9) return igemm_launch_shared_tail<64, 64, CONV_BK, 2>(al, bl, ep, M, N, K);
+  if (form == 10) return igemm_launch_shared_tail<64, 64, CONV_BK, 4>(al, bl, ep, M, N, K, 1);
+  if (form == 11) return igemm_launch_shared_tail<64, 64, CONV_BK, 4>(al, bl, ep, M, N, K);
   if (form == 6) return igemm_launch_shared_tail<64, 128, CONV_BK>(al, bl, ep, M, N, K);
   if (form == 7) return igemm_launch_shared_tail<128, 128, CONV_BK>(al, bl, ep, M, N, K);
   return igemm_launch<64, 64, CONV_BK>(al, bl, ep, M, N, K, 1);
@@ -51,7 +62,9 @@ int form_of_rule(int M, int N, int K) {
 
 namespace lh {
 // ResNet-50 at 224x224 on one card in turn, 53 such chains (before: 53 convolutions, 53 batch norms, 33 relus and 16 joins, each a pass
-// over memory): batch 32 4.28 -> 2.90 ms, batch 1 1.006 -> 0.797 ms.  What bounds it now is the convolutions themselves.
+// over memory): batch 32 4.28 -> 2.90 ms, batch 1 1.006 -> 0.797 ms; with forms 8-11 and the rows' parameters asked for ahead of the
+// operands (a round trip less per launch: batch 1 742 -> 728 us) 2.92 -> 2.74 ms and 0.794 -> 0.728 ms.  What bounds it now is the
+// convolutions themselves; at batch 1 a launch of the smallest takes 8.4 us for 4 slabs, 5 of them fixed.
 void conv2d_bn_infer_now(const float* x, const float* w, const float* bias, int N, int C, int H, int W, int K, int R, int S, int sH, int sW, int pH, int pW,
                          const float* gamma, const float* beta, const float* mean, const float* var, float eps, const float* shortcut, float* out, int relu) {
   KernelCat kc_(CAT_CONV_FWD);
@@ -80,6 +93,7 @@ void conv2d_bn_infer_now(const float* x, const float* w, const float* bias, int 
     };
     auto valid = [&](int form) {
       if ((form == 1 || form == 7) && K <= 64) return false;
+      if (form >= 8) return !g_deterministic && (form == 8 || form == 10 || g_stream_cur == g_stream_raw) && cdiv(CRS, CONV_BK) >= (form >= 10 ? 16 : 8) && cdiv(K, 64) * cdiv(cols, 64) <= 8 * (int64_t)g_num_cu;
       if (form >= 5) return !g_deterministic && g_stream_cur == g_stream_raw && CRS >= 8 * CONV_BK;
       // the convolution by itself: where its tiles are fewer than the compute units and the reduction is long enough for stream-K
       if (form == 4) return !g_deterministic && cdiv(K, 64) * cdiv(cols, 64) < g_num_cu && CRS >= 16 * CONV_BK;
@@ -89,15 +103,15 @@ void conv2d_bn_infer_now(const float* x, const float* w, const float* bias, int 
     static std::map<PlanKey, int> chosen;
     const PlanKey key = {{K, cols, CRS, H, W, sH, R | (shortcut ? 1 << 16 : 0) | (g_deterministic ? 1 << 17 : 0)}};
     int form = form_of_rule(K, cols, CRS);
-    const int forced = force_plan() >= 13 && force_plan() <= 15 ? force_plan() - 8 : force_plan();
+    const int forced = force_plan() >= 13 && force_plan() <= 19 ? force_plan() - 8 : force_plan();
     auto it = chosen.find(key);
-    if (forced >= 1 && forced <= 7 && valid(forced)) form = forced;
+    if (forced >= 1 && forced <= 11 && valid(forced)) form = forced;
     else if (it != chosen.end() && g_tune_enabled) { form = it->second; g_plans_remembered++; }
     else if (g_tune_enabled && !g_capturing && 2.0 * K * CRS * (double)cols >= g_tune_min_flop) {
       LaunchTimer timer;
       if (timer.ok) {
         float best_ms = 3.0e38f;
-        const int order[7] = {3, 2, 1, 5, 6, 7, 4};
+        const int order[11] = {3, 2, 1, 5, 6, 7, 4, 8, 9, 10, 11};
         for (int f : order) {
           if (!valid(f)) continue;
           const float ms = timer.ms([&]() { return run(f); });

@@ -34,6 +34,9 @@ CASES = [
     (2, 16, 9, 11, 64, 1, 1, 0, False, False, True, 3), (2, 16, 9, 11, 65, 3, 1, 1, True, True, True, 3), (1, 32, 7, 7, 40, 3, 2, 1, False, True, False, 2),
     (3, 64, 14, 14, 128, 3, 1, 1, False, True, True, 1), (3, 64, 14, 14, 130, 1, 1, 0, True, False, False, 1), (2, 128, 14, 14, 96, 1, 2, 0, False, True, True, 2),
     (2, 256, 7, 7, 512, 1, 1, 0, False, True, True, 13), (1, 256, 14, 14, 64, 3, 1, 1, False, False, True, 14), (2, 128, 20, 20, 136, 3, 1, 1, True, True, True, 15),
+    (1, 64, 56, 56, 64, 1, 1, 0, False, False, True, 16), (1, 16, 9, 11, 70, 3, 1, 1, True, True, True, 16), (1, 512, 7, 7, 512, 3, 1, 1, False, True, True, 17),
+    (1, 144, 14, 14, 230, 1, 1, 0, True, True, True, 18), (2, 48, 15, 13, 66, 3, 2, 1, False, False, False, 18), (1, 512, 7, 7, 512, 3, 1, 1, False, True, True, 19),
+    (1, 1008, 7, 7, 70, 1, 1, 0, False, False, True, 19),
     (1, 512, 7, 7, 512, 3, 1, 1, False, True, True, 4), (1, 512, 7, 7, 100, 1, 1, 0, False, False, False, 4),
     (2, 3, 33, 31, 64, 7, 2, 3, False, False, True, None), (2, 5, 8, 8, 7, 3, 1, 1, True, True, True, None), (8, 64, 28, 28, 256, 1, 1, 0, False, True, True, None),
     (1, 16, 1, 1, 32, 1, 1, 0, False, True, True, None),
