@@ -316,7 +316,7 @@ __global__ void __launch_bounds__(TPB) k_conv_bwd_bias(const float* __restrict__
   float acc = 0.f;
   if (VEC) {
     const int PQ4 = PQ >> 2, total = (n1 - n0) * PQ4;
-#pragma unroll 2
+#pragma unroll 4
     for (int i = threadIdx.x; i < total; i += TPB) {
       const int dn = i / PQ4, l = i - dn * PQ4;
       const int64_t o = (((int64_t)(n0 + dn) * K + k) * PQ4 + l) * 4;
@@ -344,6 +344,10 @@ __global__ void __launch_bounds__(TPB) k_conv_bwd_bias(const float* __restrict__
 }
 static void bias_grad_launch(const float* y, float* dy, float* db, int N, int K, int PQ) {
   int bslices = g_deterministic ? 1 : (int)cdiv(4 * (int64_t)g_num_cu, K);     // slices of the batch add atomically: one slice when the order must be fixed
+  // A slice is at least 16 KiB long (four loads a thread in flight): the additions to one address follow each other at 0.1 us, and a
+  // hundred of them (10 channels, 100 images of 24x24) took longer than the reading: 13.6 -> 4.4 us (SqueezeNet's 25: 203 -> 125).
+  const int64_t worth = cdiv((int64_t)N * PQ * 4, 16384);
+  if (bslices > worth) bslices = (int)worth;
   if (bslices > N) bslices = N;
   if (bslices < 1) bslices = 1;
   const int n_per = (int)cdiv(N, bslices);

@@ -123,3 +123,24 @@ def test_recorded_column_sums_leave_memory_handed_out_later_alone(on_hip):
         np.testing.assert_array_equal(d.down(held, (1 << 16,)), later)
     on_hip.graphDestroy(graph)
     on_hip.resetMallocAddr(mark)
+
+
+@pytest.mark.parametrize("N,K,P,Q", [(100, 10, 24, 24), (1, 3, 64, 64), (7, 5, 24, 25), (33, 16, 8, 16), (64, 700, 2, 2), (300, 1, 31, 33), (4097, 2, 1, 1)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_bias_gradient(on_hip, N, K, P, Q, masked):
+    """Slices of the batch around 16 KiB, masked by a relu on the way or not: sums of N P Q terms, each rounding at most 2^-24 of a partial
+    sum (below four times the terms' root sum of squares), the roundings like their square root, 8 for the rest."""
+    d = Dev(on_hip)
+    mark = on_hip.getMallocAddr()
+    rng = np.random.RandomState(N)
+    y, dy = rng.standard_normal((N, K, P, Q)).astype(np.float32), rng.standard_normal((N, K, P, Q)).astype(np.float32)
+    base = rng.standard_normal(K).astype(np.float32)
+    X, Y, G, db, dw = d.up(rng.standard_normal((N, 1, P, Q)).astype(np.float32)), d.up(y), d.up(dy), d.up(base), d.zeros(K)
+    if masked:
+        on_hip.lib.lh_unary_grad(B.RELU, Y.ptr, Y.ptr, G.ptr, G.ptr, y.size, 1, 0.0, 0.0)
+    on_hip.lib.lh_conv2d_bwd_filter(X.ptr, G.ptr, dw.ptr, db.ptr, 1.0, N, 1, P, Q, K, 1, 1, 1, 1, 0, 0); _lib.check()
+    g = np.where(y > 0, dy, 0).astype(np.float64) if masked else dy.astype(np.float64)
+    bound = (4 * np.sqrt(N * P * Q) + 8) * 2.0 ** -24 * (np.sqrt((g ** 2).sum((0, 2, 3))) + np.abs(base))
+    assert (np.abs(d.down(db, (K,)) - (base + g.sum((0, 2, 3)))) <= bound).all()
+    np.testing.assert_array_equal(d.down(G, y.shape), g.astype(np.float32))
+    on_hip.resetMallocAddr(mark)
