@@ -410,17 +410,14 @@ void lh_rnn_fwd_init(int mode, const float* x, const float* hx, const float* w, 
     if (hx) lh_sgemm(0, 1, B, H, H, 1.0f, hx + (size_t)d * B * H, H, Wih + (size_t)H * I, H, 1.0f, y + (size_t)(d == 0 ? 0 : T - 1) * B * ld + d * H, ld);
   }
   ProfScope prof_(CAT_RNN);
-  if (const size_t bytes = rnn_seq_scratch(SEQ_ELMAN, false, D, T, B, H)) {
+  if (rnn_seq_takes(SEQ_ELMAN, false, D, T, B, H)) {
     SeqLayer a = {};
     for (int d = 0; d < D; d++) {
       a.dir[d].W = w + d * dir_params(I, H) + (size_t)H * I;
       a.dir[d].b1 = a.dir[d].W + (size_t)H * H; a.dir[d].b2 = a.dir[d].b1 + H;
     }
     a.y = y; a.D = D; a.T = T; a.B = B; a.H = H; a.ld = ld; a.relu = mode == 0;
-    void* ring = lh_malloc_uninit(bytes);
-    if (ring == nullptr) return;
-    rnn_seq_run(SEQ_ELMAN, false, a, ring);
-    lh_free_top(bytes);
+    rnn_seq_run(SEQ_ELMAN, false, a);
     LH_CHECK_LAUNCH();
     return;
   }
@@ -457,14 +454,12 @@ void lh_rnn_bwd_init(int mode, const float* x, const float* hx, const float* y, 
   float* scratch = (float*)lh_malloc_uninit(bytes);
   if (scratch == nullptr) return;
   float* dpre = scratch; float* wt = dpre + n_dpre; float* colsum = wt + n_wt;
-  if (const size_t ring_bytes = rnn_seq_scratch(SEQ_ELMAN, true, D, T, B, H)) {
+  if (rnn_seq_takes(SEQ_ELMAN, true, D, T, B, H)) {
     SeqLayer a = {};
     for (int d = 0; d < D; d++) a.dir[d].W = w + d * dir_params(I, H) + (size_t)H * I;
     a.y = const_cast<float*>(y); a.dy = dy; a.dpre = dpre; a.D = D; a.T = T; a.B = B; a.H = H; a.ld = ld; a.relu = mode == 0;
-    void* ring = lh_malloc_uninit(ring_bytes);
-    if (ring == nullptr) return;
-    { ProfScope prof_(CAT_RNN); rnn_seq_run(SEQ_ELMAN, true, a, ring); }
-    lh_free_top(ring_bytes);
+    ProfScope prof_(CAT_RNN);
+    rnn_seq_run(SEQ_ELMAN, true, a);
   } else {
     for (int d = 0; d < D; d++) {
       const float* Whh = w + d * dir_params(I, H) + (size_t)H * I;

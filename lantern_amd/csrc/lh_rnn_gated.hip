@@ -287,11 +287,7 @@ void lh_rnn_gated_fwd_init(int mode, const float* x, const float* hx, const floa
   LZ_ENTER();
   lazy::rd_f(x, (int64_t)T * B * I); lazy::rd_f(w, (int64_t)D * dir_params(mode, I, H)); lazy::rd_f(hx, (int64_t)D * B * H); lazy::rd_f(cx, (int64_t)D * B * H);
   lazy::wr_f(y, (int64_t)T * B * ldh); lazy::wr_f(reserve, (int64_t)D * dir_reserve(mode, T, B, H));
-  const size_t per_dir = (size_t)B * G;
-  const size_t gh_bytes = (size_t)D * per_dir * sizeof(float);
-  float* gh_all = (float*)lh_malloc_uninit(gh_bytes);
-  if (gh_all == nullptr) return;
-  if (const size_t ring_bytes = rnn_seq_scratch(mode == 2 ? SEQ_LSTM : SEQ_GRU, false, D, T, B, H)) {
+  if (rnn_seq_takes(mode == 2 ? SEQ_LSTM : SEQ_GRU, false, D, T, B, H)) {
     SeqLayer s = {};
     for (int d = 0; d < D; d++) {
       SeqDir& p = s.dir[d];
@@ -302,14 +298,14 @@ void lh_rnn_gated_fwd_init(int mode, const float* x, const float* hx, const floa
       lh_sgemm(0, 1, T * B, G, I, 1.0f, x, I, Wih, I, 0.0f, p.act, G);
     }
     s.y = y; s.D = D; s.T = T; s.B = B; s.H = H; s.ld = ldh;
-    void* ring = lh_malloc_uninit(ring_bytes);
-    if (ring == nullptr) return;
-    rnn_seq_run(mode == 2 ? SEQ_LSTM : SEQ_GRU, false, s, ring);
-    lh_free_top(ring_bytes);
-    lh_free_top(gh_bytes);
+    rnn_seq_run(mode == 2 ? SEQ_LSTM : SEQ_GRU, false, s);
     LH_CHECK_LAUNCH();
     return;
   }
+  const size_t per_dir = (size_t)B * G;
+  const size_t gh_bytes = (size_t)D * per_dir * sizeof(float);
+  float* gh_all = (float*)lh_malloc_uninit(gh_bytes);
+  if (gh_all == nullptr) return;
   // The two directions of a bidirectional layer share nothing but the input: the reverse one runs on the library's second
   // stream beside the forward one (in line when that stream is off, while a graph is recorded or in deterministic mode).
   auto run_direction = [&](int d) {
@@ -372,8 +368,8 @@ void lh_rnn_gated_bwd_init(int mode, const float* x, const float* hx, const floa
   const size_t bytes = (size_t)D * per_dir * sizeof(float);
   float* scratch = (float*)lh_malloc_uninit(bytes);
   if (scratch == nullptr) return;
-  const size_t ring_bytes = rnn_seq_scratch(mode == 2 ? SEQ_LSTM : SEQ_GRU, true, D, T, B, H);
-  if (ring_bytes) {
+  const bool one_launch = rnn_seq_takes(mode == 2 ? SEQ_LSTM : SEQ_GRU, true, D, T, B, H);
+  if (one_launch) {
     SeqLayer s = {};
     for (int d = 0; d < D; d++) {
       SeqDir& p = s.dir[d];
@@ -383,10 +379,7 @@ void lh_rnn_gated_bwd_init(int mode, const float* x, const float* hx, const floa
       p.dgh = scratch + (size_t)d * per_dir + 2 * n_bh + 2 * (size_t)G;
     }
     s.y = const_cast<float*>(y); s.dy = dy; s.D = D; s.T = T; s.B = B; s.H = H; s.ld = ldh;
-    void* ring = lh_malloc_uninit(ring_bytes);
-    if (ring == nullptr) return;
-    rnn_seq_run(mode == 2 ? SEQ_LSTM : SEQ_GRU, true, s, ring);
-    lh_free_top(ring_bytes);
+    rnn_seq_run(mode == 2 ? SEQ_LSTM : SEQ_GRU, true, s);
   }
   // each direction has its own scratch and its own part of dw, and runs on its own stream (see the forward pass); the input
   // gradient, to which both add, is formed afterwards on the caller's stream
@@ -397,7 +390,7 @@ void lh_rnn_gated_bwd_init(int mode, const float* x, const float* hx, const floa
     float* dWih = dw + off; float* dWhh = dWih + (size_t)G * I; float* dbih = dWhh + (size_t)G * H; float* dbhh = dbih + G;
     float* act = reserve + d * dir_reserve(mode, T, B, H);
     const float* aux = act + (size_t)T * B * G;
-    for (int k = 0; k < T && !ring_bytes; k++) {
+    for (int k = 0; k < T && !one_launch; k++) {
       const int t = d == 0 ? T - 1 - k : k;                        // reverse of the forward processing order
       const int tp = d == 0 ? t - 1 : t + 1;                       // the step whose state this one consumed
       const bool has_prev = d == 0 ? t > 0 : t < T - 1;

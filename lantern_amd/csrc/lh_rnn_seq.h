@@ -19,11 +19,12 @@ struct SeqLayer {
   const float* dy; float* dpre;      // backward: incoming gradient; Elman: pre-activation gradient out, both [T, B, ld]
   int D, T, B, H, ld, relu;          // relu: the Elman layer's activation (0: tanh)
 };
-// Bytes of scratch memory such a launch needs, 0 where the layer does not run that way (see the rule in lh_rnn_seq.hip).
-size_t rnn_seq_scratch(int kind, bool backward, int D, int T, int B, int H);
+// Does the layer run that way?  (see the rule in lh_rnn_seq.hip)
+bool rnn_seq_takes(int kind, bool backward, int D, int T, int B, int H);
 // The whole recurrence on the current stream, in one launch or one per direction.
-void rnn_seq_run(int kind, bool backward, const SeqLayer& a, void* scratch);
-bool rnn_seq_setup();              // the flag word of lh_setup / lh_cleanup
+void rnn_seq_run(int kind, bool backward, const SeqLayer& a);
+extern bool g_captured_seq;        // the graph being recorded holds such a launch
+bool rnn_seq_setup();              // the ring and the flag word, for lh_setup / lh_cleanup
 void rnn_seq_release();
 bool rnn_seq_report_timeout();     // true (and an error reported) if a launch gave up waiting for a block since the last look
 }  // namespace lh

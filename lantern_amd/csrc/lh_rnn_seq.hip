@@ -5,7 +5,8 @@
 // A time step is a [B, H] x [H, gates * H] product of microseconds whose operands are 0.1 MB of state and 3 to 10 MB of weights.
 // One launch per step reads the weights again every time (no L2 keeps them over a launch) and pays for the launch.  Here every
 // block keeps the weights of its 4 to 16 hidden units in registers for the whole sequence, and what travels between the blocks
-// of a step is the state alone, through a ring of SEQ_RING slots in scratch memory:
+// of a step is the state alone, through a ring of SEQ_RING slots in memory of the library's own (not the arena's: a graph's replay
+// clears and writes the ring at the address it was recorded with, long after the arena has handed out what lay above its top then):
 //
 //   - a word of a slot is SEQ_EMPTY until the thread that owns it writes the step's value, and readers ask again until no word
 //     they were given is SEQ_EMPTY.  The word is the message: nothing depends on the order in which two words become visible,
@@ -32,6 +33,7 @@
 #include "../../include/lantern_hip.h"
 
 namespace lh {
+bool g_captured_seq = false;
 namespace {
 
 constexpr unsigned SEQ_EMPTY = 0xffffffffu;
@@ -368,6 +370,8 @@ __global__ void __launch_bounds__(256) k_seq_clear(uint4* p, int n16) {
 
 unsigned* g_flag = nullptr;
 unsigned* g_flag_dev = nullptr;
+unsigned* g_ring = nullptr;           // one, since all launches of this kind follow each other on the main stream (replays: lh_graph_launch)
+size_t g_ring_bytes = 0;
 
 // How a launch is laid out: `ct` column tiles and `units` units a block, gx * gz blocks per direction, `dirs` directions per launch,
 // `groups` groups of 16 k in a slot's tile, `nit` of them per wavefront.  Units per block: as few as leave every block a compute
@@ -401,19 +405,19 @@ Plan plan_of(int kind, bool backward, int D, int T, int B, int H) {
 size_t slot_bytes(const Plan& p) { return (size_t)p.dirs * p.gz * p.groups * 1024; }
 }  // namespace
 
-size_t rnn_seq_scratch(int kind, bool backward, int D, int T, int B, int H) {
-  if (!rnn_mfma_enabled() || g_stream_cur != g_stream_raw || g_flag_dev == nullptr) return 0;
-  if (const char* e = getenv("LH_RNN_SEQ")) if (e[0] == '0') return 0;        // (the tests' switch: one launch per time step)
+bool rnn_seq_takes(int kind, bool backward, int D, int T, int B, int H) {
+  if (!rnn_mfma_enabled() || g_stream_cur != g_stream_raw || g_ring == nullptr) return false;
+  if (const char* e = getenv("LH_RNN_SEQ")) if (e[0] == '0') return false;        // (the tests' switch: one launch per time step)
   const Plan p = plan_of(kind, backward, D, T, B, H);
-  const size_t bytes = p.ok ? SEQ_RING * slot_bytes(p) : 0;
-  return bytes <= arena_room() ? bytes : 0;
+  return p.ok && SEQ_RING * slot_bytes(p) <= g_ring_bytes;
 }
 
-void rnn_seq_run(int kind, bool backward, const SeqLayer& a, void* scratch) {
+void rnn_seq_run(int kind, bool backward, const SeqLayer& a) {
   const Plan p = plan_of(kind, backward, a.D, a.T, a.B, a.H);
   if (!p.ok) { LH_FAIL("recurrence: no launch plan for T%d B%d H%d", a.T, a.B, a.H); return; }
   SeqArgs s;
-  s.a = a; s.ring = (unsigned*)scratch; s.slot_bytes = (unsigned)slot_bytes(p); s.ring_bytes = SEQ_RING * s.slot_bytes;
+  if (g_capturing) g_captured_seq = true;
+  s.a = a; s.ring = g_ring; s.slot_bytes = (unsigned)slot_bytes(p); s.ring_bytes = SEQ_RING * s.slot_bytes;
   s.groups = p.groups; s.flag = g_flag_dev; s.spins = SEQ_SPINS;
   if (const char* e = getenv("LH_RNN_SEQ_SPINS")) s.spins = atoi(e);          // (the tests' switch: a wait that gives up at once)
   const dim3 grid((unsigned)p.gx, (unsigned)p.dirs, (unsigned)p.gz);
@@ -441,11 +445,16 @@ bool rnn_seq_setup() {
     LH_FAIL("recurrence: cannot allocate the pinned flag"); return false;
   }
   *g_flag = 0;
+  // a slot has at most four groups (the gates of a backward pass) of 1 KiB per block, and there is a compute unit for every block
+  g_ring_bytes = SEQ_RING * 4 * 1024 * (size_t)g_num_cu;
+  g_ring = (unsigned*)persistent_alloc(g_ring_bytes);
+  if (g_ring == nullptr) { LH_FAIL("recurrence: cannot allocate the ring of %zu bytes", g_ring_bytes); return false; }
   return true;
 }
 void rnn_seq_release() {
   if (g_flag) (void)hipHostFree(g_flag);
-  g_flag = g_flag_dev = nullptr;
+  persistent_free(g_ring);
+  g_flag = g_flag_dev = g_ring = nullptr;
 }
 bool rnn_seq_report_timeout() {
   if (g_flag == nullptr || *(volatile unsigned*)g_flag == 0) return false;

@@ -128,6 +128,7 @@ void prof_end(int cat) {
 }
 
 static std::vector<hipGraphExec_t> g_graphs;
+static std::vector<char> g_graph_seq;          // the graph holds a recurrence of one launch (lh_rnn_seq.hip)
 __global__ void k_set_u64(unsigned long long* p, unsigned long long keep, unsigned long long add) { *p = (keep ? *p : 0ull) + add; }
 __global__ void k_zero16(uint4* p, size_t n16) {
   size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x, st = (size_t)gridDim.x * blockDim.x;
@@ -193,7 +194,7 @@ void lh_cleanup(void) {
   multi_tensor_release();
   rnn_seq_release();
   for (auto& e : g_graphs) if (e) { (void)hipGraphExecDestroy(e); e = nullptr; }
-  g_graphs.clear(); g_capturing = false;
+  g_graphs.clear(); g_graph_seq.clear(); g_capturing = false;
   if (g_advance_pool) (void)hipFree(g_advance_pool);
   g_advance_pool = nullptr; g_capture_advance = nullptr;
   if (g_fix_cnt) (void)hipFree(g_fix_cnt);
@@ -405,7 +406,7 @@ void lh_capture_begin(void) {
   hipLaunchKernelGGL(k_set_u64, dim3(1), dim3(1), 0, g_stream, g_capture_advance, 0ull, 0ull);
   LH_CHECK_LAUNCH();
   LH_HIP(hipStreamBeginCapture(g_stream_raw, hipStreamCaptureModeThreadLocal));
-  g_capturing = true;
+  g_capturing = true; g_captured_seq = false;
   g_arena.zero_end = g_arena.top;       // a zero fill done eagerly says nothing about replays: every block handed out while recording records its own fill
 }
 int lh_capture_end(void) {
@@ -425,12 +426,20 @@ int lh_capture_end(void) {
   e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
   (void)hipGraphDestroy(graph);
   if (e != hipSuccess) { LH_FAIL("hipGraphInstantiate: %s", hipGetErrorString(e)); return -1; }
-  g_graphs.push_back(exec);
+  g_graphs.push_back(exec); g_graph_seq.push_back(g_captured_seq);
   return (int)g_graphs.size() - 1;
 }
 void lh_graph_launch(int id) {
   lazy::flush_undeclared();         // a replay reads and writes whatever its recording did (parameters included): everything deferred is brought up to date, no kept copy survives
   LH_REQUIRE(id >= 0 && id < (int)g_graphs.size() && g_graphs[id] != nullptr, "lh_graph_launch: no graph %d", id);
+  if (g_graph_seq[id] && g_stream_cur != g_stream_raw) {
+    // (its blocks need the chip together and share the library's one ring: never beside the main stream's work)
+    side_join();
+    LH_HIP(hipGraphLaunch(g_graphs[id], g_stream_raw));
+    side_wait_for_main();
+    g_side_dirty = true;
+    return;
+  }
   LH_HIP(hipGraphLaunch(g_graphs[id], g_stream));
 }
 void lh_graph_destroy(int id) {
