@@ -184,9 +184,9 @@ void lh_prof_collect(double* h_ms, int64_t* h_calls, int ncat);
  * Results are those of the calls as issued (the fused kernels give the bits of the sequences they replace wherever two
  * launches of the sequence itself agree bit for bit).  Every entry point of this header takes part; a pointer handed to
  * anything else (another library, a kernel of the caller's) must be preceded by lh_sync() AND lh_flush_deferred().
- * lh_fusion_stats: h_out[0..7] = forward chains fused, backward chains fused, optimizer calls gathered, zero fills avoided,
+ * lh_fusion_stats: h_out[0..8] = forward chains fused, backward chains fused, optimizer calls gathered, zero fills avoided,
  * zero fills done, results produced on demand, conv -> bn or bn -> + chains that ended without a relu, filter copies found
- * kept by a convolution call. */
+ * kept by a convolution call, passes of recurrent layers whose whole recurrence was one launch. */
 void lh_set_fusion(int on);
 int lh_get_fusion(void);
 void lh_flush_deferred(void);               /* everything put off is enqueued now (nothing waits) */

@@ -632,6 +632,7 @@ void on_rewind(char* new_top) {
 }
 
 }  // namespace lazy
+int64_t g_rnn_seq_runs = 0;        // (lh_rnn_seq.hip counts, lh_fusion_stats reports)
 }  // namespace lh
 
 using namespace lh;
@@ -647,6 +648,6 @@ void lh_set_fusion(int on) {
 int lh_get_fusion(void) { return lazy::g_enabled ? 1 : 0; }
 void lh_flush_deferred(void) { lazy::Scope s_; lazy::flush_all(); }
 void lh_fusion_stats(int64_t* h_out, int n) {
-  for (int i = 0; i < n; i++) h_out[i] = i < 8 ? lazy::g_stat[i] : 0;
+  for (int i = 0; i < n; i++) h_out[i] = i < 8 ? lazy::g_stat[i] : (i == 8 ? g_rnn_seq_runs : 0);
 }
 }

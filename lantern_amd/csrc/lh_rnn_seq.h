@@ -23,6 +23,7 @@ struct SeqLayer {
 bool rnn_seq_takes(int kind, bool backward, int D, int T, int B, int H);
 // The whole recurrence on the current stream, in one launch or one per direction.
 void rnn_seq_run(int kind, bool backward, const SeqLayer& a);
+extern int64_t g_rnn_seq_runs;     // passes run (or recorded) that way since the library was loaded
 extern bool g_captured_seq;        // the graph being recorded holds such a launch
 bool rnn_seq_setup();              // the ring and the flag word, for lh_setup / lh_cleanup
 void rnn_seq_release();

@@ -417,6 +417,7 @@ void rnn_seq_run(int kind, bool backward, const SeqLayer& a) {
   if (!p.ok) { LH_FAIL("recurrence: no launch plan for T%d B%d H%d", a.T, a.B, a.H); return; }
   SeqArgs s;
   if (g_capturing) g_captured_seq = true;
+  g_rnn_seq_runs++;
   s.a = a; s.ring = g_ring; s.slot_bytes = (unsigned)slot_bytes(p); s.ring_bytes = SEQ_RING * s.slot_bytes;
   s.groups = p.groups; s.flag = g_flag_dev; s.spins = SEQ_SPINS;
   if (const char* e = getenv("LH_RNN_SEQ_SPINS")) s.spins = atoi(e);          // (the tests' switch: a wait that gives up at once)

@@ -1,6 +1,8 @@
 """The recurrence as one launch (lh_rnn_seq.hip) against the same layer with one launch per time step (LH_RNN_SEQ=0), which
 test_parity_ops.py holds to the oracle: at the edges of its tiles (16 units, 16 batch rows, groups of 16 k dealt to 4 wavefronts),
 of its register forms and of its launch plans; replayed from a graph; and when a block gives up waiting."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -9,6 +11,12 @@ from tests.util import Dev
 
 pytestmark = pytest.mark.gpu
 GATES = {0: 1, 1: 1, 2: 4, 3: 3}          # relu, tanh, LSTM, GRU
+
+
+def _one_launch_passes(be):
+    stats = (ctypes.c_int64 * 9)()
+    be.lib.lh_fusion_stats(stats, 9)
+    return stats[8]
 
 
 def _layer(d, mode, T, B, I, H, bidir, init, seed=5):
@@ -46,12 +54,14 @@ def test_one_launch_against_one_per_step(hip_backend, monkeypatch, case):
     the next with a factor around one (weights of norm about 0.7), and T <= 14 of them add up: below 1e-5 of the result's rms, four
     times which is allowed."""
     d = Dev(hip_backend)
-    mark = d.be.getMallocAddr()
+    mark, before = d.be.getMallocAddr(), _one_launch_passes(d.be)
     got = _layer(d, *case)
     d.be.resetMallocAddr(mark)
+    assert _one_launch_passes(d.be) == before + 2, "forward and backward are one launch each"
     monkeypatch.setenv("LH_RNN_SEQ", "0")
     want = _layer(d, *case)
     d.be.resetMallocAddr(mark)
+    assert _one_launch_passes(d.be) == before + 2
     for name, a, b in zip(("y", "dx", "dw"), got, want):
         rms = float(np.sqrt(np.mean(np.square(b, dtype=np.float64))))
         assert np.isfinite(a).all() and np.abs(a - b).max() <= 4e-5 * (np.abs(b).max() + rms), name
