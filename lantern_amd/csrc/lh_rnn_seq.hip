@@ -19,7 +19,8 @@
 //
 // All blocks of a launch have to be resident together: at most one block per compute unit is launched, on the main stream only
 // (so no second launch of this kind, nor the command list's, runs beside it), and whatever else holds a compute unit ends by
-// itself.  A wait is bounded all the same; a block whose wait runs out says so in a pinned word and goes on without waiting.
+// itself.  Every step's waits are bounded all the same; a wavefront whose wait runs out says so in a pinned word and goes on without waiting,
+// to the end of the sequence.
 //
 // What bounds it is latency: of an Elman step's 2.4 us (B 32, H 800) the matrix instructions take 0.7, the rest is a word's way out
 // (a write-through store) and in (polls of 0.7 us a round), LDS and the activation.  Per step, one launch per step -> now, B 32,
@@ -39,7 +40,7 @@ namespace {
 constexpr unsigned SEQ_EMPTY = 0xffffffffu;
 constexpr int SEQ_RING = 4;
 constexpr int SEQ_COHERENT = 17;             // cache policy bits of the buffer instructions: sc0 | sc1
-constexpr int SEQ_SPINS = 4000000;           // polls before a block gives up: seconds, where a real wait is microseconds
+constexpr int SEQ_SPINS = 4000000;           // polls in one step before a wavefront gives up: seconds, where a real wait is microseconds
 constexpr int RS = 68;                       // floats of LDS per accumulator register of a tile (64 lanes, padded: the finishing threads read it transposed)
 
 struct SeqArgs {
@@ -190,6 +191,7 @@ __global__ void __launch_bounds__(256, 1) k_rnn_seq_fwd(const SeqArgs s) {
   int spins = s.spins;
   SeqProduct<NIT, CT> m;
   for (int step = 0; step < T; step++) {
+    if (spins >= 0) spins = s.spins;              // the bound is a step's
     const int tt = d == 0 ? step : T - 1 - step;
     float* red = red_all[step & 1];
     const bool use = step > 0 || (KIND != SEQ_ELMAN && p.h0 != nullptr);
@@ -305,6 +307,7 @@ __global__ void __launch_bounds__(256, 1) k_rnn_seq_bwd(const SeqArgs s) {
   float carry = 0.f;                    // LSTM: cell gradient, GRU: dh * z
   SeqProduct<NIT, 1> m;
   for (int k = 0; k < T; k++) {
+    if (spins >= 0) spins = s.spins;              // the bound is a step's
     const int tt = d == 0 ? T - 1 - k : k;
     const int64_t row = (int64_t)tt * B + b;
     float* red = red_all[k & 1];

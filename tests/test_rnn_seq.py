@@ -161,3 +161,18 @@ def test_a_wait_that_runs_out_is_reported_once(hip_backend, monkeypatch):
     y = be.rnn_forward(1, X, W, 40, 33, 8, 64, False)
     assert np.isfinite(d.down(y, (40, 33, 64))).all()
     be.resetMallocAddr(mark)
+
+
+def test_the_bound_is_a_waits_own(hip_backend, monkeypatch):
+    """60000 steps, many of them with a poll or more that finds words missing, pass under a bound that every single wait stays far below."""
+    d, T, B, I, H = Dev(hip_backend), 60000, 1, 4, 256
+    be, rng = d.be, np.random.RandomState(7)
+    mark = be.getMallocAddr()
+    X, W = d.up(rng.standard_normal((T, B, I)).astype(np.float32)), d.up((rng.standard_normal(H * I + H * H + 2 * H) * 0.1).astype(np.float32))
+    dy, dx, dw = d.up(rng.standard_normal((T, B, H)).astype(np.float32)), d.zeros(T * B * I), d.zeros(W.n)
+    monkeypatch.setenv("LH_RNN_SEQ_SPINS", "1000")
+    y = be.rnn_forward(1, X, W, T, B, I, H, False)
+    be.sync()
+    be.rnn_backward(1, X, y, dy, W, dx, dw, T, B, I, H, False)
+    be.sync()
+    be.resetMallocAddr(mark)
