@@ -324,8 +324,13 @@ void lh_bn_bwd(const float* x, const float* dy, const float* gamma, const float*
  *   W_ih[H,I], W_hh[H,H], b_ih[H], b_hh[H] (NNModule.scala:378-390), forward direction first.
  * lh_rnn_bwd: dx = beta_dx*dx + ... (dx may be NULL), dw += ...; takes T*B*D*H + D*H*H + ... floats of
  * scratch from the top of the arena and releases them before returning.
- * The recurrence runs one kernel per time step; for 16-byte aligned operands and 64 <= H <= 2048 that kernel uses the matrix
- * instructions (LH_RNN_MFMA=0 in the environment keeps the vector form everywhere). */
+ * The recurrence is one launch for the whole sequence where it is long enough (12 steps, 4 for the gated modes), runs on the main
+ * stream and its blocks fit the compute units at once.  Those blocks wait for each other, so such layers expect the card to
+ * themselves as far as other processes go: with a second process running them on it a bounded wait may run out, which the next
+ * lh_sync or lh_d2h reports as an error (that layer's results are incomplete), and from then until lh_cleanup every layer takes one
+ * kernel per time step, the form of all other layers; LH_RNN_SEQ=0 in the environment takes that form from the start.  For 16-byte
+ * aligned operands and 64 <= H <= 2048 the kernel per step uses the matrix instructions (LH_RNN_MFMA=0 in the environment keeps
+ * the vector form everywhere). */
 void lh_rnn_fwd(int mode, const float* x, const float* w, float* y, int T, int B, int I, int H, int bidir);
 void lh_rnn_bwd(int mode, const float* x, const float* y, const float* dy, const float* w, float* dx, float beta_dx, float* dw,
                 int T, int B, int I, int H, int bidir);

@@ -18,8 +18,10 @@
 //     it has waited for its own stores (s_waitcnt vmcnt(0) behind every step's first loads), so no reader can meet an old value.
 //
 // All blocks of a launch have to be resident together: at most one block per compute unit is launched, on the main stream only
-// (so no second launch of this kind, nor the command list's, runs beside it), and whatever else holds a compute unit ends by
-// itself.  Every step's waits are bounded all the same; a wavefront whose wait runs out says so in a pinned word and goes on without waiting,
+// (so no second launch of this kind, nor the command list's, runs beside it), and whatever else of this process holds a compute unit
+// ends by itself.  A second process that runs such layers on the same card can hold the units this launch still needs while it waits
+// for those this one holds: the waits then run out, and from the first one that did the process keeps one launch
+// per step (graphs recorded before hold what they hold).  Every step's waits are bounded all the same; a wavefront whose wait runs out says so in a pinned word and goes on without waiting,
 // to the end of the sequence.
 //
 // What bounds it is latency: of an Elman step's 2.4 us (B 32, H 800) the matrix instructions take 0.7, the rest is a word's way out
@@ -373,6 +375,7 @@ __global__ void __launch_bounds__(256) k_seq_clear(uint4* p, int n16) {
 
 unsigned* g_flag = nullptr;
 unsigned* g_flag_dev = nullptr;
+bool g_given_up = false;              // a wait has run out: the card is shared, or something else keeps blocks from it
 unsigned* g_ring = nullptr;           // one, since all launches of this kind follow each other on the main stream (replays: lh_graph_launch)
 size_t g_ring_bytes = 0;
 
@@ -410,7 +413,12 @@ size_t slot_bytes(const Plan& p) { return (size_t)p.dirs * p.gz * p.groups * 102
 
 bool rnn_seq_takes(int kind, bool backward, int D, int T, int B, int H) {
   if (!rnn_mfma_enabled() || g_stream_cur != g_stream_raw || g_ring == nullptr) return false;
-  if (const char* e = getenv("LH_RNN_SEQ")) if (e[0] == '0') return false;        // (the tests' switch: one launch per time step)
+  if (*(volatile unsigned*)g_flag != 0) g_given_up = true;
+  if (const char* e = getenv("LH_RNN_SEQ")) {        // (the tests' switch: 0 one launch per time step, 1 the one launch again after a wait that ran out)
+    if (e[0] == '0') return false;
+    if (e[0] == '1') g_given_up = false;
+  }
+  if (g_given_up) return false;
   const Plan p = plan_of(kind, backward, D, T, B, H);
   return p.ok && SEQ_RING * slot_bytes(p) <= g_ring_bytes;
 }
@@ -448,7 +456,7 @@ bool rnn_seq_setup() {
   if (hipHostMalloc((void**)&g_flag, 64, hipHostMallocDefault) != hipSuccess || hipHostGetDevicePointer((void**)&g_flag_dev, g_flag, 0) != hipSuccess) {
     LH_FAIL("recurrence: cannot allocate the pinned flag"); return false;
   }
-  *g_flag = 0;
+  *g_flag = 0; g_given_up = false;
   // a slot has at most four groups (the gates of a backward pass) of 1 KiB per block, and there is a compute unit for every block
   g_ring_bytes = SEQ_RING * 4 * 1024 * (size_t)g_num_cu;
   g_ring = (unsigned*)persistent_alloc(g_ring_bytes);
@@ -463,7 +471,8 @@ void rnn_seq_release() {
 bool rnn_seq_report_timeout() {
   if (g_flag == nullptr || *(volatile unsigned*)g_flag == 0) return false;
   *g_flag = 0;
-  LH_FAIL("recurrent layer: a block waited too long for the others; the layer's results are incomplete");
+  g_given_up = true;
+  LH_FAIL("recurrent layer: a block waited too long for the others; the layer's results are incomplete (the layers that follow take one launch per time step)");
   return true;
 }
 }  // namespace lh

@@ -19,6 +19,14 @@ def _one_launch_passes(be):
     return stats[8]
 
 
+def _waited(be):
+    """An event the host has waited for, without the error check of lh_sync."""
+    e = be.lib.lh_event_create()
+    be.lib.lh_event_record(e)
+    assert be.lib.lh_event_elapsed_ms(e, e) == 0
+    return e
+
+
 def _layer(d, mode, T, B, I, H, bidir, init, seed=5):
     """Forward and backward of one layer; everything it returns or leaves behind."""
     be, rng, D, G = d.be, np.random.RandomState(seed), 2 if bidir else 1, GATES[mode] * H
@@ -158,8 +166,27 @@ def test_a_wait_that_runs_out_is_reported_once(hip_backend, monkeypatch):
         be.sync()
     monkeypatch.delenv("LH_RNN_SEQ_SPINS")
     be.sync()
-    y = be.rnn_forward(1, X, W, 40, 33, 8, 64, False)
-    assert np.isfinite(d.down(y, (40, 33, 64))).all()
+    before = _one_launch_passes(be)
+    y = be.rnn_forward(1, X, W, 40, 33, 8, 64, False)           # one launch per time step from here on
+    assert np.isfinite(d.down(y, (40, 33, 64))).all() and _one_launch_passes(be) == before
+    monkeypatch.setenv("LH_RNN_SEQ", "1")
+    be.rnn_forward(1, X, W, 40, 33, 8, 64, False)
+    monkeypatch.delenv("LH_RNN_SEQ")
+    again = be.rnn_forward(1, X, W, 40, 33, 8, 64, False)
+    assert _one_launch_passes(be) == before + 2
+    np.testing.assert_allclose(d.down(again, (40, 33, 64)), d.down(y, (40, 33, 64)), atol=1e-5)
+    monkeypatch.setenv("LH_RNN_SEQ_SPINS", "0")            # given up by a call that no wait has reported yet: the next one knows
+    be.rnn_forward(1, X, W, 40, 33, 8, 64, False)
+    monkeypatch.delenv("LH_RNN_SEQ_SPINS")
+    be.lib.lh_event_destroy(_waited(be))
+    be.rnn_forward(1, X, W, 40, 33, 8, 64, False)
+    assert _one_launch_passes(be) == before + 3
+    with pytest.raises(LanternHipError, match="waited too long"):
+        be.sync()
+    monkeypatch.setenv("LH_RNN_SEQ", "1")
+    be.rnn_forward(1, X, W, 40, 33, 8, 64, False)
+    assert _one_launch_passes(be) == before + 4
+    be.sync()
     be.resetMallocAddr(mark)
 
 
