@@ -28,6 +28,7 @@
 #include "lh_infer.h"
 #include <string.h>
 #include <algorithm>
+#include <set>
 #include <vector>
 
 namespace lh {
@@ -54,9 +55,14 @@ struct Unwritten {
   int kind; char* dst; size_t bytes;
   const float* src; const float* y; int64_t n;                                           // V_MASK: dst = y > 0 ? src : 0
   const float* x; const float* gamma; const float* beta; const float* sm; const float* si; int N, C, HW;   // V_BN_OUT: dst = bn(x); V_BN_INFER: the same from running statistics (sm, si: mean, variance)
-  float eps; ConvArgs conv;                                                              // V_CONV: dst = conv(x)
+  float eps; ConvArgs conv;                                                              // V_CONV: dst = conv(x); V_BN_INFER: the convolution in front of it
 };
 static std::vector<Unwritten> g_unwritten;
+// Filters whose inference chain has left out a result that was asked for after all (read, or its operands overwritten while it
+// could still be read: a program with fixed buffers, one that flushes before it rewinds): producing it runs the convolution
+// again, which costs more than the chain saves.  Their calls run as issued from then on, until the filter is released.
+static std::set<const char*> g_wanted;
+static const size_t WANTED_MAX = 1 << 16;
 
 struct FwdRecord { const float* y; const float* x; const float* bias; int64_t n; };   // y = relu(bn(x)) as the fused kernels compute it
 static std::vector<FwdRecord> g_records;
@@ -197,9 +203,10 @@ static void produce(const Unwritten& v) {
   if (v.kind == V_MASK) { rd(v.src, (size_t)v.n * 4); rd(v.y, (size_t)v.n * 4); }
   else if (v.kind == V_CONV) { const ConvArgs& c = v.conv; rd(c.x, (size_t)c.N * c.C * c.H * c.W * 4); rd(c.w, (size_t)c.K * c.C * c.R * c.S * 4); if (c.bias) rd(c.bias, (size_t)c.K * 4); }
   else { rd(v.x, (size_t)v.n * 4); }
+  const ConvArgs& c = v.conv;
+  if (v.kind == V_CONV || v.kind == V_BN_INFER) { if (g_wanted.size() >= WANTED_MAX) g_wanted.clear(); g_wanted.insert((const char*)c.w); }
   Replay r_;
   g_stat[ST_RECIPES]++;
-  const ConvArgs& c = v.conv;
   if (v.kind == V_MASK) mask_relu((float*)v.dst, v.src, v.y, v.n);
   else if (v.kind == V_CONV) lh_conv2d_fwd(c.x, c.w, c.bias, c.y, c.N, c.C, c.H, c.W, c.K, c.R, c.S, c.sH, c.sW, c.pH, c.pW);
   else if (v.kind == V_BN_INFER) bn_infer_now(v.x, v.gamma, v.beta, v.sm, v.si, v.eps, nullptr, (float*)v.dst, 0, v.N, v.C, v.HW);
@@ -315,7 +322,7 @@ static void launch_infer_chain(const Parked& p, int relu, const float* shortcut,
   g_unwritten.push_back(v);
   if (shortcut) {
     Unwritten u{}; u.kind = V_BN_INFER; u.dst = (char*)b.y; u.bytes = (size_t)b.n * 4; u.n = b.n;
-    u.x = b.x; u.gamma = b.gamma; u.beta = b.beta; u.sm = b.rm; u.si = b.rv; u.eps = b.eps; u.N = b.N; u.C = b.C; u.HW = b.HW;
+    u.x = b.x; u.gamma = b.gamma; u.beta = b.beta; u.sm = b.rm; u.si = b.rv; u.eps = b.eps; u.N = b.N; u.C = b.C; u.HW = b.HW; u.conv = c;
     g_unwritten.push_back(u);
   }
   g_stat[ST_FUSED_FWD]++;
@@ -435,6 +442,7 @@ bool park_bn_infer(const float* x, const float* gamma, const float* beta, const 
   if (!can_park() || g_capturing || conv2d_bn_infer_now == nullptr || bn_infer_now == nullptr || !x || !gamma || !beta || !mean || !var || !y) return false;
   const int64_t n = (int64_t)N * C * HW;
   if (!(g_p.kind == P_CONV && g_p.conv.y == x && g_p.conv.N == N && g_p.conv.K == C && (int64_t)g_p.conv.P * g_p.conv.Q == HW)) return false;
+  if (g_wanted.count((const char*)g_p.conv.w)) return false;
   BnArgs b = {x, gamma, beta, const_cast<float*>(mean), const_cast<float*>(var), y, nullptr, nullptr, N, C, HW, eps, 0.f, n};
   b.infer = true;
   if (over_conv_operands(g_p.conv, y, n) || over_channels(b, y, n)) return false;
@@ -588,7 +596,7 @@ bool gather_update(int mode, float* x, float* d, float* v, float lr, float mu, f
   return true;
 }
 void forget_forward_records() { g_records.clear(); }
-void reset() { g_p = Parked(); g_zero.clear(); g_unwritten.clear(); g_records.clear(); layouts_drop(); g_busy = false; g_replay = false; }
+void reset() { g_p = Parked(); g_zero.clear(); g_unwritten.clear(); g_records.clear(); g_wanted.clear(); layouts_drop(); g_busy = false; g_replay = false; }
 
 // An inference chain's result that stays, made from what is released, is produced before it goes.
 static void produce_from_released(const char* from) {
@@ -599,8 +607,10 @@ static void produce_from_released(const char* from) {
     if (gone && v.dst < from) { const Unwritten copy = v; g_unwritten.erase(g_unwritten.begin() + i); produce(copy); i = 0; } else i++;
   }
 }
+void filters_released(const char* from) { if (!g_wanted.empty()) g_wanted.erase(g_wanted.lower_bound(from), g_wanted.end()); }
 void arena_released(char* from) {
   if (!g_unwritten.empty()) produce_from_released(from);
+  filters_released(from);
   if (!g_layouts.empty()) layouts_released(from);
   while (!g_zero.empty() && g_zero.back().p >= from) g_zero.pop_back();
   for (size_t i = 0; i < g_unwritten.size();) {

@@ -21,8 +21,8 @@
 // (so no second launch of this kind, nor the command list's, runs beside it), and whatever else of this process holds a compute unit
 // ends by itself.  A second process that runs such layers on the same card can hold the units this launch still needs while it waits
 // for those this one holds: the waits then run out, and from the first one that did the process keeps one launch
-// per step (graphs recorded before hold what they hold).  Every step's waits are bounded all the same; a wavefront whose wait runs out says so in a pinned word and goes on without waiting,
-// to the end of the sequence.
+// per step (graphs recorded before hold what they hold).  Every step's waits are bounded all the same; a wavefront whose wait runs
+// out says so in a pinned word and goes on without waiting, to the end of the sequence.
 //
 // What bounds it is latency: of an Elman step's 2.4 us (B 32, H 800) the matrix instructions take 0.7, the rest is a word's way out
 // (a write-through store) and in (polls of 0.7 us a round), LDS and the activation.  Per step, one launch per step -> now, B 32,

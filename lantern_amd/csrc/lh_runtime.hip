@@ -3,6 +3,7 @@
 // API:453-473 (myGpuMalloc / myGpuFree), CUB:37-107 (toGPU / toCPU).
 #include "lh_common.h"
 #include "lh_arena.h"
+#include "lh_infer.h"
 #include "lh_rnn_seq.h"
 #include <stdarg.h>
 #include <string.h>
@@ -241,14 +242,15 @@ void lh_free_top(size_t bytes) {
   if (lazy::g_busy) {
     if (lazy::g_depth == 0) { LZ_ENTER(); }       // a caller's pop (myGpuFree): nothing parked may still want the block
     lazy::arena_released(g_heap + g_arena.top - need);
-  }
+  } else lazy::filters_released(g_heap + g_arena.top - need);
   (void)arena_pop(g_arena, bytes);
 }
 size_t lh_mark(void) { return g_arena.top; }
 void lh_rewind(size_t mark) {
   LH_REQUIRE(mark <= g_arena.top && (mark & 255) == 0, "lh_rewind(%zu): not a mark at or below the top (%zu)", mark, g_arena.top);
   LZ_SCOPE();
-  if (lazy::g_busy) lazy::on_rewind(g_heap + mark);     // zero fills and unread results of what is released are simply dropped
+  if (!lazy::g_busy) lazy::filters_released(g_heap + mark);
+  else lazy::on_rewind(g_heap + mark);                  // zero fills and unread results of what is released are simply dropped
   side_join();      // what is handed out again must not be in use on the side stream
   (void)arena_rewind(g_arena, mark);
 }

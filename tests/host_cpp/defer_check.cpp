@@ -101,7 +101,8 @@ static void sim_pop(size_t bytes) {                   // lh_free_top: scratch ta
 // ---- simulated kernels: any deterministic functions will do, as long as a fused form computes what its parts compute ------
 static const int N_ = 2, C_ = 4, HW_ = 24, NE = N_ * C_ * HW_;      // every activation: 192 floats = 768 bytes (a "large" block)
 static inline int chan(int i) { return (i / HW_) % C_; }
-static void k_conv(const float* x, const float* w, const float* bias, float* y) { for (int i = 0; i < NE; i++) { float a = bias ? bias[chan(i)] : 0.f; for (int k = 0; k < 3; k++) a += x[(i + 7 * k) % NE] * w[(chan(i) + k) % 12]; y[i] = a; } g_kernels++; }
+static long long g_convs = 0;             // forward convolutions among them
+static void k_conv(const float* x, const float* w, const float* bias, float* y) { g_convs++; for (int i = 0; i < NE; i++) { float a = bias ? bias[chan(i)] : 0.f; for (int k = 0; k < 3; k++) a += x[(i + 7 * k) % NE] * w[(chan(i) + k) % 12]; y[i] = a; } g_kernels++; }
 static void k_conv_bwd_data(const float* dy, const float* w, float* dx, float beta) { for (int i = 0; i < NE; i++) { float a = 0.f; for (int k = 0; k < 3; k++) a += dy[(i + NE - 7 * k) % NE] * w[(chan((i + NE - 7 * k) % NE) + k) % 12]; dx[i] = (beta != 0.f ? dx[i] : 0.f) + a; } g_kernels++; }
 static void k_conv_bwd_filter(const float* x, const float* dy, float* dw, float beta) { for (int j = 0; j < 12; j++) { float a = 0.f; for (int i = 0; i < NE; i++) for (int k = 0; k < 3; k++) if ((chan(i) + k) % 12 == j) a += dy[i] * x[(i + 7 * k) % NE]; dw[j] = (beta != 0.f ? dw[j] : 0.f) + a; } g_kernels++; }
 namespace lh {

@@ -98,6 +98,7 @@ static void infer_program(uint64_t seed, bool enabled, std::vector<float>& trace
   image.assign(g_heap, g_heap + g_arena.top);
 }
 
+#ifndef DEFER_INFER_NO_MAIN          // (defer_infer_launches.cpp has one of its own)
 int main(int argc, char** argv) {
   const int programs = argc > 1 ? atoi(argv[1]) : 2000;
   const uint64_t seed0 = argc > 2 ? (uint64_t)atoll(argv[2]) : 1;
@@ -118,3 +119,4 @@ int main(int argc, char** argv) {
   free(g_heap);
   return 0;
 }
+#endif

@@ -13,20 +13,31 @@ from lantern_amd import backend as B
 HERE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "host_cpp")
 
 
-@pytest.mark.parametrize("seed", [1, 2])
-def test_chains_give_what_the_calls_as_issued_give(tmp_path, seed):
+def _build_host_check(tmp_path, name):
     if shutil.which("g++") is None:
         pytest.skip("no host C++ compiler")
-    exe = str(tmp_path / "defer_infer_check")
+    exe = str(tmp_path / name)
     r = subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-fsanitize=address,undefined", "-fno-sanitize-recover=all", "-x", "c++", "-I", os.path.join(HERE, "fake_hip"),
-                        "-o", exe, os.path.join(HERE, "defer_infer_check.cpp")], capture_output=True, text=True)
+                        "-o", exe, os.path.join(HERE, name + ".cpp")], capture_output=True, text=True)
     if r.returncode != 0 and "cannot find" in r.stderr:
         pytest.skip("the sanitizer runtimes are not installed: " + r.stderr[-300:])
     assert r.returncode == 0, r.stderr[-3000:]
     env = dict(os.environ)
     env.pop("LD_PRELOAD", None)
+    return exe, env
+
+
+@pytest.mark.parametrize("seed", [1, 2])
+def test_chains_give_what_the_calls_as_issued_give(tmp_path, seed):
+    exe, env = _build_host_check(tmp_path, "defer_infer_check")
     r = subprocess.run([exe, "2000", str(seed)], capture_output=True, text=True, timeout=600, env=env)
     assert r.returncode == 0 and "identical" in r.stdout and " 0 chains" not in r.stdout, (r.stdout + r.stderr)[-3000:]
+
+
+def test_chains_cost_no_more_launches_than_the_calls_as_issued(tmp_path):
+    exe, env = _build_host_check(tmp_path, "defer_infer_launches")
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=600, env=env)
+    assert r.returncode == 0 and "defer_infer_launches: ok" in r.stdout, (r.stdout + r.stderr)[-3000:]
 
 
 # N, C, H, W, K, filter, stride, padding, bias, join, relu, launch form (LH_FORCE_PLAN; None: the measured one)
