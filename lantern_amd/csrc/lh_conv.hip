@@ -486,12 +486,8 @@ static bool launch_plan(int plan, const AL& al, const BL& bl, const EP& ep, int 
   if (plan == 1) return launch_rounds<128, 128, 64, 64>(al, bl, ep, M, N, K);
   if (plan == 2) return launch_rounds<64, 128, 64, 64>(al, bl, ep, M, N, K);
   if (plan == 3) return igemm_launch<64, 64, CONV_BK>(al, bl, ep, M, N, K, 1);
-  const int64_t t128 = cdiv(M, 128) * cdiv(N, 128), t64 = cdiv(M, 64) * cdiv(N, 128);
   const int workers = 2 * g_num_cu;
-  const bool few = (M > 64 ? t128 : t64) < 6 * (int64_t)g_num_cu;
-  const int64_t slabs = cdiv(K, CONV_BK);
-  // long reductions only: a worker's share must span many slabs for the per-segment set-up to pay off
-  if (!g_deterministic && few && slabs >= 64 && slabs * (M > 64 ? t128 : t64) >= 48 * (int64_t)workers && (ep.beta == 1.f || zero_out != nullptr || prezeroed)) {
+  if (stream_k_rule(M, N, K) && (ep.beta == 1.f || zero_out != nullptr || prezeroed)) {
     if (ep.beta == 0.f && !prezeroed) lh_fill(zero_out, 0.f, zero_n);
     g_launch_partial = true;
     if (M > 64) return igemm_launch<128, 128, CONV_BK>(al, bl, ep, M, N, K, 1, workers);
@@ -549,10 +545,7 @@ struct StatLayout { int col1, g_main, slots_main, g_rem, slots_rem; int sliced =
 // launches nothing) for shapes that take the stream-K path, whose tiles are finished by several blocks.
 template <class AL, class BL>
 static bool plan_tiles_stats(int M, int N, int K, StatLayout& L, int& bm, int& bn, int force = 0 /* 1-3: the tile of launch plan 1-3; 5-7: 64x64 / 64x128 / 128x128 tiles with the last ones sliced; 8-10: launch plans 16-18 */) {
-  const int64_t t128 = cdiv(M, 128) * cdiv(N, 128), t64 = cdiv(M, 64) * cdiv(N, 128);
-  const bool few = (M > 64 ? t128 : t64) < 6 * (int64_t)g_num_cu;
-  const int64_t slabs = cdiv(K, CONV_BK);
-  if (!g_deterministic && few && slabs >= 64 && slabs * (M > 64 ? t128 : t64) >= 48 * (int64_t)(2 * g_num_cu)) return false;
+  if (stream_k_rule(M, N, K)) return false;
   TilePick tp = pick_tile_conv(M, N, K);
   if ((force == 1 || force == 7) && M > 64) tp = {128, 128}; else if (force == 2 || force == 6) tp = {64, 128}; else if (force == 3 || force == 5 || force >= 8) tp = {64, 64};
   L.groups = force >= 8 && deep_ok(M, N, K, force == 9 ? 4 : 2) ? (force == 9 ? 4 : 2) : 1;

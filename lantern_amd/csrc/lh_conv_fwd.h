@@ -153,6 +153,12 @@ static inline TilePick pick_tile_conv(int M, int N, int K) {
   if (K <= 512) return {64, 64};
   return pick_tile(M, N);
 }
+// The built-in rule's other half: few tiles over a long reduction run stream-K (a worker's share must span many slabs for the
+// per-segment set-up to pay off).
+static inline bool stream_k_rule(int M, int N, int K) {
+  const int64_t tiles = M > 64 ? cdiv(M, 128) * cdiv(N, 128) : cdiv(M, 64) * cdiv(N, 128), slabs = cdiv(K, CONV_BK);
+  return !g_deterministic && tiles < 6 * (int64_t)g_num_cu && slabs >= 64 && slabs * tiles >= 48 * (int64_t)(2 * g_num_cu);
+}
 // The filter in the layout a launch reads: the library's kept copy (written now if it is stale), or, where none is kept,
 // scratch from the arena top that the caller pops behind the launch (stream order keeps that safe).
 struct FilterCopy { float* p = nullptr; size_t scratch = 0; };

@@ -40,7 +40,8 @@ struct EpiConvBn : EpiConvOut {
 
 // Launch forms: 1-3 whole tiles 128x128, 64x128, 64x64; 5-7 the last tiles of 64x64 / 64x128 / 128x128 sliced along the reduction
 // (igemm_launch_shared_tail); 8-11 64x64 tiles on blocks of two groups of wavefronts, whole and sliced, and of four, whole and sliced;
-// 4 the convolution by itself (any of its launch plans, stream-K among them), then the pass over it.
+// 4 the convolution by itself (any of its launch plans, stream-K among them), then the pass over it.  Channel counts that are no multiple of
+// the slab's depth: 2, 3 and 4.
 template <class AL, class BL>
 bool launch_form(int form, const AL& al, const BL& bl, const EpiConvBn& ep, int M, int N, int K) {
   if (form == 1) return igemm_launch<128, 128, CONV_BK>(al, bl, ep, M, N, K, 1);
@@ -75,34 +76,17 @@ void conv2d_bn_infer_now(const float* x, const float* w, const float* bias, int 
   EpiConvBn ep;
   static_cast<EpiConvOut&>(ep) = make_epi(out, bias, K, d.P, d.Q, 0.f);
   ep.relu = relu; ep.gamma = gamma; ep.shift = beta; ep.mean = mean; ep.var = var; ep.eps = eps; ep.shortcut = shortcut;
-  bool ok;
-  if (C % CONV_BK == 0 && ((uintptr_t)w & 15) == 0) {
-    // tap-major reduction order; a 1x1 filter already has that layout
-    FilterCopy fc;
-    fc.p = const_cast<float*>(w);
-    const int prm[LAYOUT_PRM] = {K, C, RS};
-    if (RS > 1 && !filter_copy(fc, w, wbytes, LAYOUT_KRSC, prm, wbytes)) return;
-    LoadPlainK<true> al; al.base = fc.p; al.nbytes = wbytes; al.ld = CRS;
-    LoadConvFwdTapB bl; bl.base = x; bl.nbytes = xbytes; bl.C = C; bl.H = H; bl.W = W; bl.sH = sH; bl.sW = sW; bl.pH = pH; bl.pW = pW; bl.HW = H * W;
-    bl.dPQ.init(PQ); bl.dQ.init(d.Q); bl.dC.init(C); bl.dS.init(S);
-    auto run = [&](int form) {
-      if (form != 4) return launch_form(form, al, bl, ep, K, cols, CRS);
-      lh_conv2d_fwd(x, w, bias, out, N, C, H, W, K, R, S, sH, sW, pH, pW);
-      if (!failed()) bn_infer_now(out, gamma, beta, mean, var, eps, shortcut, out, relu, N, K, PQ);
-      return !failed();
-    };
-    auto valid = [&](int form) {
-      if ((form == 1 || form == 7) && K <= 64) return false;
-      if (form >= 8) return !g_deterministic && (form == 8 || form == 10 || g_stream_cur == g_stream_raw) && cdiv(CRS, CONV_BK) >= (form >= 10 ? 16 : 8) && cdiv(K, 64) * cdiv(cols, 64) <= 8 * (int64_t)g_num_cu;
-      if (form >= 5) return !g_deterministic && g_stream_cur == g_stream_raw && CRS >= 8 * CONV_BK;
-      // the convolution by itself: where its tiles are fewer than the compute units and the reduction is long enough for stream-K
-      if (form == 4) return !g_deterministic && cdiv(K, 64) * cdiv(cols, 64) < g_num_cu && CRS >= 16 * CONV_BK;
-      return true;
-    };
-    // the form is measured once per shape (the launch overwrites `out` and nothing else, so repeating it is harmless) and remembered
+  // Form 4: the convolution by itself, then the pass over it.  (`form` below: the rule's, where nothing is measured)
+  auto parts = [&]() {
+    lh_conv2d_fwd(x, w, bias, out, N, C, H, W, K, R, S, sH, sW, pH, pW);
+    if (!failed()) bn_infer_now(out, gamma, beta, mean, var, eps, shortcut, out, relu, N, K, PQ);
+    return !failed();
+  };
+  // The form is measured once per shape (the launch overwrites `out` and nothing else, so repeating it is harmless) and remembered.
+  // false: reported.
+  auto run_measured = [&](int loader, int form, auto valid, auto run) {
     static std::map<PlanKey, int> chosen;
-    const PlanKey key = {{K, cols, CRS, H, W, sH, R | (shortcut ? 1 << 16 : 0) | (g_deterministic ? 1 << 17 : 0)}};
-    int form = form_of_rule(K, cols, CRS);
+    const PlanKey key = {{K, cols, CRS, H, W, sH, R | (shortcut ? 1 << 16 : 0) | (g_deterministic ? 1 << 17 : 0) | loader << 18}};
     const int forced = force_plan() >= 13 && force_plan() <= 19 ? force_plan() - 8 : force_plan();
     auto it = chosen.find(key);
     if (forced >= 1 && forced <= 11 && valid(forced)) form = forced;
@@ -115,21 +99,56 @@ void conv2d_bn_infer_now(const float* x, const float* w, const float* bias, int 
         for (int f : order) {
           if (!valid(f)) continue;
           const float ms = timer.ms([&]() { return run(f); });
-          if (ms < 0.f || failed()) { if (fc.scratch) lh_free_top(fc.scratch); return; }
+          if (ms < 0.f || failed()) return false;
           if (ms < best_ms * 0.98f) { best_ms = ms; form = f; }
         }
         chosen[key] = form; g_plans_measured++;
         if (getenv("LH_TUNE_VERBOSE")) fprintf(stderr, "conv + bn (running) K%d N%d CRS%d H%d: form %d, %.4f ms\n", K, cols, CRS, H, form, best_ms);
       }
     }
-    ok = run(form);
+    return run(form);
+  };
+  bool ok;
+  if (C % CONV_BK == 0 && ((uintptr_t)w & 15) == 0) {
+    // tap-major reduction order; a 1x1 filter already has that layout
+    FilterCopy fc;
+    fc.p = const_cast<float*>(w);
+    const int prm[LAYOUT_PRM] = {K, C, RS};
+    bool copied = RS == 1;
+    LoadPlainK<true> al; al.base = fc.p; al.nbytes = wbytes; al.ld = CRS;
+    LoadConvFwdTapB bl; bl.base = x; bl.nbytes = xbytes; bl.C = C; bl.H = H; bl.W = W; bl.sH = sH; bl.sW = sW; bl.pH = pH; bl.pW = pW; bl.HW = H * W;
+    bl.dPQ.init(PQ); bl.dQ.init(d.Q); bl.dC.init(C); bl.dS.init(S);
+    auto valid = [&](int form) {
+      if ((form == 1 || form == 7) && K <= 64) return false;
+      if (form >= 8) return !g_deterministic && (form == 8 || form == 10 || g_stream_cur == g_stream_raw) && cdiv(CRS, CONV_BK) >= (form >= 10 ? 16 : 8) && cdiv(K, 64) * cdiv(cols, 64) <= 8 * (int64_t)g_num_cu;
+      if (form >= 5) return !g_deterministic && g_stream_cur == g_stream_raw && CRS >= 8 * CONV_BK;
+      // the convolution by itself, where stream-K may win more than the pass behind it costs: fewer tiles than compute units, or a long
+      // reduction (512 -> 512 channels 3x3 over 14x14, batch 32: 231 -> 219 us; without measuring, 7x7 over 7x7 to 4096 1798 -> 1091)
+      if (form == 4) return !g_deterministic && (CRS >= 64 * CONV_BK || (cdiv(K, 64) * cdiv(cols, 64) < g_num_cu && CRS >= 16 * CONV_BK));
+      return true;
+    };
+    ok = run_measured(0, stream_k_rule(K, cols, CRS) ? 4 : form_of_rule(K, cols, CRS), valid, [&](int form) {
+      if (form == 4) return parts();
+      if (!copied && !filter_copy(fc, w, wbytes, LAYOUT_KRSC, prm, wbytes)) return false;
+      copied = true; al.base = fc.p;
+      return launch_form(form, al, bl, ep, K, cols, CRS);
+    });
     if (fc.scratch) lh_free_top(fc.scratch);
   } else {
+    // Any other channel count: whole 64x64 and 64x128 tiles, or the parts with the convolution's own choice of plans (stream-K, tiles of
+    // 32 rows, groups of wavefronts).  A whole tile by rule, its filter loaded 4 bytes at a time -> the measured form | the parts:
+    // 100 -> 100 channels 3x3 over 7x7, batch 64 80.6 -> 27.8 | 29.8 us, 20 -> 50 channels 5x5 over 28x28, batch 1 31.3 -> 15.7 | 17.9.
     LoadConvFwdB bl; bl.base = x; bl.nbytes = xbytes; bl.C = C; bl.H = H; bl.W = W; bl.sH = sH; bl.sW = sW; bl.pH = pH; bl.pW = pW; bl.HW = H * W;
     bl.dPQ.init(PQ); bl.dQ.init(d.Q); bl.dRS.init(RS); bl.dS.init(S);
-    LoadPlainK<false> al; al.base = w; al.nbytes = wbytes; al.ld = CRS;
-    if (form_of_rule(K, cols, CRS) == 3) ok = igemm_launch<64, 64, CONV_BK>(al, bl, ep, K, cols, CRS, 1);
-    else ok = igemm_launch<64, 128, CONV_BK>(al, bl, ep, K, cols, CRS, 1);
+    auto valid = [&](int form) { return form == 2 || form == 3 || (form == 4 && !g_deterministic); };
+    auto with = [&](const auto& al, int loader) {
+      return run_measured(loader, form_of_rule(K, cols, CRS), valid, [&](int form) {
+        if (form == 4) return parts();
+        return form == 3 ? igemm_launch<64, 64, CONV_BK>(al, bl, ep, K, cols, CRS, 1) : igemm_launch<64, 128, CONV_BK>(al, bl, ep, K, cols, CRS, 1);
+      });
+    };
+    if (CRS % 4 == 0 && ((uintptr_t)w & 15) == 0) { LoadPlainK<true> al; al.base = w; al.nbytes = wbytes; al.ld = CRS; ok = with(al, 1); }
+    else { LoadPlainK<false> al; al.base = w; al.nbytes = wbytes; al.ld = CRS; ok = with(al, 2); }
   }
   if (!ok) return;
   LH_CHECK_LAUNCH();

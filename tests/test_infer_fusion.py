@@ -51,6 +51,9 @@ CASES = [
     (1, 512, 7, 7, 512, 3, 1, 1, False, True, True, 4), (1, 512, 7, 7, 100, 1, 1, 0, False, False, False, 4),
     (2, 3, 33, 31, 64, 7, 2, 3, False, False, True, None), (2, 5, 8, 8, 7, 3, 1, 1, True, True, True, None), (8, 64, 28, 28, 256, 1, 1, 0, False, True, True, None),
     (1, 16, 1, 1, 32, 1, 1, 0, False, True, True, None),
+    (2, 20, 12, 12, 50, 5, 1, 0, True, False, True, 2), (2, 20, 12, 12, 65, 5, 1, 0, False, True, True, 3), (2, 20, 12, 12, 50, 5, 1, 0, False, True, False, 4),
+    (3, 9, 13, 11, 130, 3, 2, 1, False, True, True, 2), (3, 9, 13, 11, 64, 3, 1, 1, True, True, True, 3), (3, 9, 13, 11, 33, 3, 1, 1, True, False, True, 4),
+    (2, 100, 7, 7, 100, 3, 1, 1, False, True, True, None), (4, 200, 7, 7, 30, 3, 1, 1, False, False, True, None), (1, 512, 14, 14, 96, 3, 1, 1, False, True, True, 4),
 ]
 
 
@@ -127,6 +130,30 @@ def test_chain_against_its_parts(on_hip, monkeypatch, case):
         err = (torch.from_numpy(g).double().reshape(v.shape) - v).abs()
         bound = 8 * 2.0 ** -24 * (mag + y.abs() + 1) if name == "convolution" else tol
         assert bool((err <= bound).all()), (name, float((err / bound).max()))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", [(3, 20, 30, 30, 51, 5, 1, 0), (5, 9, 31, 29, 30, 3, 1, 1)], ids=lambda c: "-".join(map(str, c)))
+def test_the_form_is_measured_for_any_channel_count(on_hip, case):
+    """Channel counts that are no multiple of the slab's depth: among the forms is the convolution by itself with its own choice of
+    plans, which a whole tile under a long reduction is far behind (100 -> 100 channels over 7x7: 81 against 31 us)."""
+    import ctypes
+    be, lib = on_hip, on_hip.lib
+    measured, remembered = ctypes.c_int64(), ctypes.c_int64()
+    seen = []
+    mark = be.getMallocAddr()
+    for _ in range(2):
+        _chain(be, lib, B, case + (False, False, True, None))
+        be.resetMallocAddr(mark)
+        lib.lh_tune_counters(ctypes.byref(measured), ctypes.byref(remembered))
+        seen.append((measured.value, remembered.value))
+    lib.lh_set_fusion(0)
+    _chain(be, lib, B, case + (False, False, True, None))          # the convolution's own plan
+    lib.lh_set_fusion(1)
+    be.resetMallocAddr(mark)
+    lib.lh_tune_counters(ctypes.byref(measured), ctypes.byref(remembered))
+    assert measured.value == seen[1][0] == seen[0][0], "the first chain measured its form and, for one of the forms, the convolution's plan"
+    assert seen[1][1] > seen[0][1]
 
 
 @pytest.mark.gpu
