@@ -398,48 +398,83 @@ static void launch_bcast_op(int op, const float* a, const float* b, float* out, 
   else hipLaunchKernelGGL((k_bcast_op<int64_t>), dim3(stream_grid(n, TPB * 4)), dim3(TPB), 0, g_stream, op, a, b, out, D, n);
 }
 
-// small[j] += sum_r sign * big[r, j] over [rows, cols] (a bias gradient).  A block sums a slice of the rows for 64 columns, four rows at
+// small[j] += sum_r sign * big[r, j] over [rows, cols] (a bias gradient).  A block sums a slice of the rows for 64 columns, Q rows at
 // a time, 8 loads a thread in flight; more than one slice: into their own rows of `partial`, which k_col_finish adds up in order.
-__global__ void __launch_bounds__(TPB) k_col_sums(float* small, float* __restrict__ partial, const float* __restrict__ big, int rows, int cols, int per, float sign) {
-  __shared__ float sm[4][64];
-  const int l = threadIdx.x & 63, q = threadIdx.x >> 6, j = blockIdx.x * 64 + l;
+// A thread's eight sums are added in pairs after 16 rows each, so that no chain of additions is longer than 16 or a 2048th of the rows
+// (a wavefront per column, the first form of this sum, had chains of a 64th): its error against 64 bits is never above that form's.
+__device__ __forceinline__ float pair_sum(const float (&a)[8]) { return ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7])); }
+template <int Q>
+__global__ void __launch_bounds__(64 * Q) k_col_sums(float* small, float* __restrict__ partial, const float* __restrict__ big, int rows, int cols, int per, float sign) {
+  __shared__ float sm[Q][64];
+  const int l = threadIdx.x & 63, q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = blockIdx.x * 64 + l;
   const int r0 = blockIdx.y * per, r1 = min(rows, r0 + per);
-  float acc[2] = {0.f, 0.f};
+  float total = 0.f;
   if (j < cols) {
     const float* p = big + j;
-    int r = r0 + q;
-    for (; r + 28 < r1; r += 32) {
-      float v[8];
+    for (int r = r0 + q; r < r1;) {
+      float acc[8];
 #pragma unroll
-      for (int e = 0; e < 8; e++) v[e] = p[(int64_t)(r + 4 * e) * cols];
+      for (int e = 0; e < 8; e++) acc[e] = 0.f;
+      const int stop = min(r1, r + 16 * 8 * Q);
+      for (; r + 7 * Q < stop; r += 8 * Q) {
+        float v[8];
 #pragma unroll
-      for (int e = 0; e < 8; e++) acc[e & 1] += v[e];
+        for (int e = 0; e < 8; e++) v[e] = p[(int64_t)(r + e * Q) * cols];
+#pragma unroll
+        for (int e = 0; e < 8; e++) acc[e] += v[e];
+      }
+      if (r < stop) {                    // (the last rows of the slice: fewer than 8 a thread)
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) { v[e] = 0.f; if (r + e * Q < stop) v[e] = p[(int64_t)(r + e * Q) * cols]; }
+#pragma unroll
+        for (int e = 0; e < 8; e++) acc[e] += v[e];
+        r += 8 * Q;
+      }
+      total += pair_sum(acc);
     }
-    for (; r < r1; r += 4) acc[0] += p[(int64_t)r * cols];
   }
-  sm[q][l] = acc[0] + acc[1];
+  sm[q][l] = total;
   __syncthreads();
-  if (q == 0 && j < cols) {
-    const float t = (sm[0][l] + sm[1][l]) + (sm[2][l] + sm[3][l]);
-    if (partial) partial[(int64_t)blockIdx.y * cols + j] = t;
-    else small[j] += sign * t;
-  }
+  if (q != 0 || j >= cols) return;
+  float t[Q];
+#pragma unroll
+  for (int i = 0; i < Q; i++) t[i] = sm[i][l];
+#pragma unroll
+  for (int h = Q / 2; h > 0; h >>= 1)
+#pragma unroll
+    for (int i = 0; i < h; i++) t[i] += t[i + h];
+  if (partial) partial[(int64_t)blockIdx.y * cols + j] = t[0];
+  else small[j] += sign * t[0];
 }
 __global__ void __launch_bounds__(TPB) k_col_finish(float* small, const float* __restrict__ partial, int slices, int cols, float sign) {
   const int j = blockIdx.x * TPB + threadIdx.x;
   if (j >= cols) return;
-  float acc = 0.f;
-#pragma unroll 8
-  for (int s = 0; s < slices; s++) acc += partial[(int64_t)s * cols + j];
-  small[j] += sign * acc;
+  float acc[8];
+#pragma unroll
+  for (int e = 0; e < 8; e++) acc[e] = 0.f;
+  for (int s = 0; s < slices; s += 8) {
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] = partial[(int64_t)min(s + e, slices - 1) * cols + j];
+#pragma unroll
+    for (int e = 0; e < 8; e++) acc[e] += s + e < slices ? v[e] : 0.f;
+  }
+  small[j] += sign * pair_sum(acc);
 }
-// true: done.  8192x4096 191 -> 25 us, 64x1000 3.6 -> 3.1 us against a wavefront per column reading one element of a row at a time.
+// true: done.  Slices: a second launch costs 2.5 us, which a block of 16 wavefronts over up to 2048 rows is done in (2048x1000 6.6 us, 2
+// slices 6.6); beyond, a block per compute unit, four slices where there are columns enough (4096x50257 187 -> 172 us), 512 rows a block.
+// 8192x4096 23 us, 64x1000 4.0, 256x1000 4.1, 1000000x4 25 (a wavefront per column reading one element of a row at a time: 178, 4.2,
+// 5.0, 8306; with 8 chains a slice and slices of 64 rows in place of the pairs: 23, 3.7, 6.8, 133).
 static bool col_sums(float* small, const float* big, int rows, int cols, float sign) {
   const int gx = (int)cdiv(cols, 64);
-  int slices = (int)cdiv(4 * (int64_t)g_num_cu, gx);
-  if (slices > rows / 64) slices = rows / 64;             // at least 16 rows a thread
-  if (slices < 1) slices = 1;
-  if (slices > 64) slices = 64;
+  int slices = 1;
+  if (rows > 2048) {
+    slices = (int)cdiv(g_num_cu, gx);
+    if (slices < 4) slices = rows / 1024 < 4 ? rows / 1024 : 4;
+    if (slices > rows / 512) slices = rows / 512;
+    if (slices > 256) slices = 256;
+  }
   const int per = (int)cdiv(rows, slices);
   slices = (int)cdiv(rows, per);
   bool side = false;
@@ -450,7 +485,10 @@ static bool col_sums(float* small, const float* big, int rows, int cols, float s
     partial = (float*)scratch_take(bytes, side);
     if (partial == nullptr) return true;                  // (reported)
   }
-  hipLaunchKernelGGL(k_col_sums, dim3((unsigned)gx, (unsigned)slices), dim3(TPB), 0, g_stream, small, partial, big, rows, cols, per, sign);
+  const dim3 grid((unsigned)gx, (unsigned)slices);
+  if (rows > 128) hipLaunchKernelGGL(k_col_sums<16>, grid, dim3(1024), 0, g_stream, small, partial, big, rows, cols, per, sign);
+  else if (rows > 16) hipLaunchKernelGGL(k_col_sums<4>, grid, dim3(256), 0, g_stream, small, partial, big, rows, cols, per, sign);      // (31x4096: 3.8 | 4.2 us)
+  else hipLaunchKernelGGL(k_col_sums<1>, grid, dim3(64), 0, g_stream, small, partial, big, rows, cols, per, sign);                   // (4x1000000: 5.8 | 7.5)
   if (bytes) {
     hipLaunchKernelGGL(k_col_finish, dim3((unsigned)cdiv(cols, TPB)), dim3(TPB), 0, g_stream, small, (const float*)partial, slices, cols, sign);
     scratch_give(bytes, side);

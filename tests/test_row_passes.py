@@ -103,6 +103,28 @@ def test_broadcast_over_rows(on_hip, full, small, op):
     on_hip.resetMallocAddr(mark)
 
 
+@pytest.mark.parametrize("rows,cols", [(64, 1000), (65, 300), (129, 77), (256, 1000), (2048, 512), (2049, 64), (4096, 4096), (5000, 800), (1024, 65536)])
+def test_column_sums_round_no_more_than_a_wavefront_per_column(on_hip, rows, cols):
+    """The order of the sum this one replaced: 64 lanes that add up every 64th row, then halves of the lanes onto each other.  The rms of
+    the error against 64 bits over the columns (a statistic of `cols` samples: 4 / sqrt(cols) wide) is not above that order's."""
+    d = Dev(on_hip)
+    mark = on_hip.getMallocAddr()
+    a = np.random.RandomState(rows).standard_normal((rows, cols)).astype(np.float32)
+    exact = np.sum(a, 0, dtype=np.float64)
+    t, A = d.zeros(cols), d.up(a)
+    on_hip.lib.lh_bcast_update(B.ADD, t.ptr, B._ints((1, cols)), A.ptr, B._ints((rows, cols)), 2); _lib.check()
+    got = d.down(t, (cols,))
+    lanes = np.zeros((64, cols), np.float32)
+    for r in range(0, rows, 64):
+        part = a[r:r + 64]
+        lanes[:len(part)] += part
+    while len(lanes) > 1:
+        lanes = lanes[:len(lanes) // 2] + lanes[len(lanes) // 2:]
+    rms = lambda e: float(np.sqrt(np.mean(np.square(e))))      # noqa: E731
+    assert rms(got - exact) <= rms(lanes[0] - exact) * (1 + 4 / np.sqrt(cols)), (rms(got - exact), rms(lanes[0] - exact))
+    on_hip.resetMallocAddr(mark)
+
+
 def test_recorded_column_sums_leave_memory_handed_out_later_alone(on_hip):
     """A graph's replay runs what was recorded at the addresses it was recorded with: partial sums kept above the arena's top would land
     in what the program has allocated there since."""
