@@ -349,17 +349,20 @@ __global__ void __launch_bounds__(TPB) k_bcast_op(int op, const float* a, const 
 }
 
 // out[r, j] = a[r, j] op b[j] over [rows, cols] (a bias added to rows): a thread owns the columns (VEC: four neighbouring ones) of a
-// few rows and reads b once.  8192x4096 in place 141 -> 46 us, 64x1000 5.1 -> 2.3 us against one thread per element with its
-// index taken apart.
-template <bool VEC>
-__global__ void __launch_bounds__(TPB) k_bcast_rows(int op, const float* a, const float* __restrict__ b, float* out, int rows, int cols, int per) {
-  const int j = (blockIdx.x * TPB + threadIdx.x) * (VEC ? 4 : 1);
-  if (j >= cols) return;
-  const int r0 = blockIdx.y * per, r1 = min(rows, r0 + per);
+// few rows and reads b once.  SIDE, rows of at most half a block: `across` threads a row, TPB / across rows side by side, neighbouring
+// threads at neighbouring addresses across the rows' ends (1000000x4 17.8 us one thread per element, 166 one row a block, 6.2 side by
+// side; 1000000x29 96.9, 147, 36.6; 262144x64 58, 60, 21).
+// 8192x4096 in place 141 -> 46 us, 64x1000 5.1 -> 2.3 us against one thread per element with its index taken apart.
+template <bool VEC, bool SIDE>
+__global__ void __launch_bounds__(TPB) k_bcast_rows(int op, const float* a, const float* __restrict__ b, float* out, int rows, int cols, int across, int per) {
+  const int side = SIDE ? TPB / across : 1, at = SIDE ? threadIdx.x / across : 0;
+  const int j = (blockIdx.x * TPB + (threadIdx.x - at * across)) * (VEC ? 4 : 1);
+  if (at >= side || j >= cols) return;
+  const uint32_t r0 = blockIdx.y * (uint32_t)(per * side) + at, r1 = min((uint32_t)rows, (blockIdx.y + 1) * (uint32_t)(per * side));      // (below 2^31 and a block)
   if (VEC) {
     const float4 bv = *reinterpret_cast<const float4*>(b + j);
 #pragma unroll 4
-    for (int r = r0; r < r1; r++) {
+    for (uint32_t r = r0; r < r1; r += side) {
       const int64_t i = (int64_t)r * cols + j;
       const float4 v = *reinterpret_cast<const float4*>(a + i);
       *reinterpret_cast<float4*>(out + i) = make_float4(bop(op, v.x, bv.x), bop(op, v.y, bv.y), bop(op, v.z, bv.z), bop(op, v.w, bv.w));
@@ -367,7 +370,7 @@ __global__ void __launch_bounds__(TPB) k_bcast_rows(int op, const float* a, cons
   } else {
     const float bv = b[j];
 #pragma unroll 4
-    for (int r = r0; r < r1; r++) { const int64_t i = (int64_t)r * cols + j; out[i] = bop(op, a[i], bv); }
+    for (uint32_t r = r0; r < r1; r += side) { const int64_t i = (int64_t)r * cols + j; out[i] = bop(op, a[i], bv); }
   }
 }
 // Is the second operand of D the trailing dimensions of the first, which has the output's shape?  (rows, cols: the two parts)
@@ -388,12 +391,14 @@ static void launch_bcast_op(int op, const float* a, const float* b, float* out, 
   int rows, cols;
   if (out != b && rows_of(D, D.sb, D.sa, rows, cols)) {
     const bool vec = cols % 4 == 0 && (((uintptr_t)a | (uintptr_t)b | (uintptr_t)out) & 15) == 0;
-    const int gx = (int)cdiv(cols, vec ? 4 * TPB : TPB);
-    int per = (int)cdiv((int64_t)rows * gx, 8 * (int64_t)g_num_cu);
-    if (cdiv(rows, per) > 65535) per = (int)cdiv(rows, 65535);
-    const dim3 grid((unsigned)gx, (unsigned)cdiv(rows, per));
-    if (vec) hipLaunchKernelGGL((k_bcast_rows<true>), grid, dim3(TPB), 0, g_stream, op, a, b, out, rows, cols, per);
-    else hipLaunchKernelGGL((k_bcast_rows<false>), grid, dim3(TPB), 0, g_stream, op, a, b, out, rows, cols, per);
+    const int threads = (int)cdiv(cols, vec ? 4 : 1), gx = (int)cdiv(threads, TPB), across = threads <= TPB / 2 ? threads : TPB, side = TPB / across;
+    const int64_t groups = cdiv(rows, side);
+    int per = (int)cdiv(groups * gx, 8 * (int64_t)g_num_cu);
+    if (cdiv(groups, per) > 65535) per = (int)cdiv(groups, 65535);
+    const dim3 grid((unsigned)gx, (unsigned)cdiv(groups, per));
+#define GO(V, S) hipLaunchKernelGGL((k_bcast_rows<V, S>), grid, dim3(TPB), 0, g_stream, op, a, b, out, rows, cols, across, per)
+    if (side > 1) { if (vec) GO(true, true); else GO(false, true); } else { if (vec) GO(true, false); else GO(false, false); }
+#undef GO
   } else if (n <= 0x7fffffff) hipLaunchKernelGGL((k_bcast_op<uint32_t>), dim3(stream_grid(n, TPB * 4)), dim3(TPB), 0, g_stream, op, a, b, out, D, n);
   else hipLaunchKernelGGL((k_bcast_op<int64_t>), dim3(stream_grid(n, TPB * 4)), dim3(TPB), 0, g_stream, op, a, b, out, D, n);
 }

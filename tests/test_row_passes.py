@@ -61,7 +61,9 @@ def test_softmax_of_rows_without_a_finite_maximum(on_hip):
 
 
 SHAPES = [((7, 5), (5,)), ((1000, 3), (3,)), ((64, 1000), (1000,)), ((2, 4096), (4096,)), ((8192, 66), (66,)), ((3, 5, 4, 8), (4, 8)), ((3, 5, 4, 8), (5, 4, 8)),
-          ((6, 5, 4, 4), (5, 1, 1)), ((2, 1, 9), (9,)), ((70000, 4), (4,)), ((33, 257), (257,))]
+          ((6, 5, 4, 4), (5, 1, 1)), ((2, 1, 9), (9,)), ((70000, 4), (4,)), ((33, 257), (257,)),
+          # rows side by side in a block: up to 128 threads a row (of one element or of four), remainders of rows and of threads
+          ((1031, 2), (2,)), ((600001, 3), (3,)), ((2051, 127), (127,)), ((2051, 128), (128,)), ((2051, 129), (129,)), ((517, 508), (508,)), ((517, 512), (512,)), ((517, 516), (516,)), ((3, 6), (6,))]
 
 
 @pytest.mark.parametrize("full,small", SHAPES)
