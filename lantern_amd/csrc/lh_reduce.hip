@@ -167,6 +167,12 @@ __global__ void __launch_bounds__(TPB) k_softmax_rows_grad(const float* y, const
 #pragma unroll
   for (int e = 0; e < E; e++) acc += LOG ? g[e] : g[e] * v[e];
   acc = row_sum<NW>(acc, sm);
+  // (the exponentials stay here: moved up under their loads' conditions, each load is waited for before the next is asked for; 32768x1000
+  // 110 -> 88 us)
+  if (LOG) {
+#pragma unroll
+    for (int e = 0; e < E; e++) asm volatile("" : "+v"(v[e]));
+  }
 #pragma unroll
   for (int e = 0; e < E; e++) {
     const int j = t + 64 * NW * e;
@@ -184,6 +190,7 @@ static bool softmax_plan(int64_t rows, int c, F go) {
   if (four) { if (per <= 4) go(std::integral_constant<int, 4>(), std::integral_constant<int, 4>(), grid); else go(std::integral_constant<int, 4>(), std::integral_constant<int, SM_REG>(), grid); }
   else if (per <= 1) go(std::integral_constant<int, 1>(), std::integral_constant<int, 1>(), grid);
   else if (per <= 4) go(std::integral_constant<int, 1>(), std::integral_constant<int, 4>(), grid);
+  else if (per <= 8) go(std::integral_constant<int, 1>(), std::integral_constant<int, 8>(), grid);
   else go(std::integral_constant<int, 1>(), std::integral_constant<int, SM_REG>(), grid);
   return true;
 }
