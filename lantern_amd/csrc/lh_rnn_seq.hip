@@ -383,7 +383,8 @@ size_t g_ring_bytes = 0;
 // `groups` groups of 16 k in a slot's tile, `nit` of them per wavefront.  Units per block: as few as leave every block a compute
 // unit of its own (a step's matrix instructions, 0.7 us per column tile at H 800, are then spread widest); both directions in one
 // launch where they fit, one after the other where only one does.  Layers that fit neither way (more than 16 batch rows times 16
-// units per compute unit: B 64 from H 1024 on, LSTM backward above H 800, whose weights exceed the registers) keep one launch per step.
+// units per compute unit: B 64 from H 1024 on; LSTM backward above H 800, where the largest form built, 50 groups a wavefront and 436
+// of 512 registers, ends) keep one launch per step.
 struct Plan { bool ok; int ct, units, nit, gx, gz, dirs, groups; };
 Plan plan_of(int kind, bool backward, int D, int T, int B, int H) {
   Plan p{};
@@ -404,6 +405,10 @@ Plan plan_of(int kind, bool backward, int D, int T, int B, int H) {
       p.dirs = dirs;
       p.ok = (int64_t)p.gx * p.gz * dirs <= g_num_cu;
     }
+  // Two launches one after the other in place of both directions at once: a forward pass of few units has too little to do in each
+  // (one launch per step | two of these: B 512, H 128 T 12 54.6 | 57.7 us, T 24 98.1 | 99.6, T 48 185 | 179; B 1024, H 64 T 24 94.6 | 98.0, T 48
+  // 172 | 175, T 100 342 | 337; B 256, H 256 T 12 60.8 | 59.0).
+  if (kind == SEQ_ELMAN && !backward && p.dirs < D && ug <= 8 && T < 48) p.ok = false;
   const int most = backward ? (kind == SEQ_ELMAN ? 32 : 50) : (p.ct >= 4 ? 13 : 16);
   if (p.nit > (kind == SEQ_ELMAN ? 32 : most)) p.ok = false;
   return p;

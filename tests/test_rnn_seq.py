@@ -75,6 +75,23 @@ def test_one_launch_against_one_per_step(hip_backend, monkeypatch, case):
         assert np.isfinite(a).all() and np.abs(a - b).max() <= 4e-5 * (np.abs(b).max() + rms), name
 
 
+@pytest.mark.parametrize("T,B,H,forward,backward", [(47, 512, 128, 0, 1), (48, 512, 128, 1, 1), (12, 256, 129, 1, 1), (12, 256, 128, 1, 1), (11, 2, 16, 0, 0)])
+def test_which_layers_are_one_launch(hip_backend, T, B, H, forward, backward):
+    """Both directions of a tanh layer: below 12 steps, and forward below 48 where the directions follow each other and have 128 units
+    at most, one launch per step is faster."""
+    d = Dev(hip_backend)
+    be = d.be
+    mark = be.getMallocAddr()
+    X, W = d.zeros(T * B * 4), d.zeros(2 * (H * 4 + H * H + 2 * H))
+    before = _one_launch_passes(be)
+    y = be.rnn_forward(1, X, W, T, B, 4, H, True)
+    assert _one_launch_passes(be) == before + forward
+    be.rnn_backward(1, X, y, d.zeros(T * B * 2 * H), W, d.zeros(X.n), d.zeros(W.n), T, B, 4, H, True)
+    assert _one_launch_passes(be) == before + forward + backward
+    be.sync()
+    be.resetMallocAddr(mark)
+
+
 @pytest.mark.parametrize("mode", [1, 2, 3])
 def test_not_a_number_stays_in_its_batch_row(hip_backend, mode):
     """One NaN in the input of a sample (with the bits the ring uses for an empty word): that sample's later states are NaN, no
