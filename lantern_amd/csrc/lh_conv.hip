@@ -464,8 +464,8 @@ static bool launch_plan(int plan, const AL& al, const BL& bl, const EP& ep, int 
   if (plan == 13) return igemm_launch_shared_tail<64, 64, CONV_BK>(al, bl, ep, M, N, K);
   if (plan == 14) return igemm_launch_shared_tail<64, 128, CONV_BK>(al, bl, ep, M, N, K);
   if (plan == 15) return igemm_launch_shared_tail<128, 128, CONV_BK>(al, bl, ep, M, N, K);
-  if (plan == 16) return igemm_launch_shared_tail<64, 64, CONV_BK, 2>(al, bl, ep, M, N, K, 1);
-  if (plan == 17) return igemm_launch_shared_tail<64, 64, CONV_BK, 4>(al, bl, ep, M, N, K, 1);
+  if (plan == 16) return igemm_launch_shared_tail<64, 64, CONV_BK, 2, 1>(al, bl, ep, M, N, K);
+  if (plan == 17) return igemm_launch_shared_tail<64, 64, CONV_BK, 4, 1>(al, bl, ep, M, N, K);
   if (plan == 18) return igemm_launch_shared_tail<64, 64, CONV_BK, 2>(al, bl, ep, M, N, K);
   if (plan >= 11) {
     g_launch_partial = true;
@@ -570,8 +570,8 @@ template <class AL, class BL>
 static bool launch_tiles_stats(const AL& al, const BL& bl, EpiConvOutStats ep, int M, int N, int K, const StatLayout& L, int bm, int bn) {
   ep.slotBase = 0;
   bool ok;
-  if (L.groups == 4) return igemm_launch_shared_tail<64, 64, CONV_BK, 4>(al, bl, ep, M, N, K, 1);
-  if (L.groups == 2) return igemm_launch_shared_tail<64, 64, CONV_BK, 2>(al, bl, ep, M, N, K, L.sliced ? 8 : 1);
+  if (L.groups == 4) return igemm_launch_shared_tail<64, 64, CONV_BK, 4, 1>(al, bl, ep, M, N, K);
+  if (L.groups == 2) return L.sliced ? igemm_launch_shared_tail<64, 64, CONV_BK, 2>(al, bl, ep, M, N, K) : igemm_launch_shared_tail<64, 64, CONV_BK, 2, 1>(al, bl, ep, M, N, K);
   if (L.sliced) return bm == 128 ? igemm_launch_shared_tail<128, 128, CONV_BK>(al, bl, ep, M, N, K) : (bn == 128 ? igemm_launch_shared_tail<64, 128, CONV_BK>(al, bl, ep, M, N, K) : igemm_launch_shared_tail<64, 64, CONV_BK>(al, bl, ep, M, N, K));
   if (bm == 128) ok = igemm_launch<128, 128, CONV_BK>(al, bl, ep, M, N, K, 1, 0, 0, L.col1);
   else if (bn == 128) ok = igemm_launch<64, 128, CONV_BK>(al, bl, ep, M, N, K, 1, 0, 0, L.col1);

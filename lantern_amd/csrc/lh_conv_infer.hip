@@ -47,9 +47,9 @@ bool launch_form(int form, const AL& al, const BL& bl, const EpiConvBn& ep, int 
   if (form == 1) return igemm_launch<128, 128, CONV_BK>(al, bl, ep, M, N, K, 1);
   if (form == 2) return igemm_launch<64, 128, CONV_BK>(al, bl, ep, M, N, K, 1);
   if (form == 5) return igemm_launch_shared_tail<64, 64, CONV_BK>(al, bl, ep, M, N, K);
-  if (form == 8) return igemm_launch_shared_tail<64, 64, CONV_BK, 2>(al, bl, ep, M, N, K, 1);
+  if (form == 8) return igemm_launch_shared_tail<64, 64, CONV_BK, 2, 1>(al, bl, ep, M, N, K);
   if (form == 9) return igemm_launch_shared_tail<64, 64, CONV_BK, 2>(al, bl, ep, M, N, K);
-  if (form == 10) return igemm_launch_shared_tail<64, 64, CONV_BK, 4>(al, bl, ep, M, N, K, 1);
+  if (form == 10) return igemm_launch_shared_tail<64, 64, CONV_BK, 4, 1>(al, bl, ep, M, N, K);
   if (form == 11) return igemm_launch_shared_tail<64, 64, CONV_BK, 4>(al, bl, ep, M, N, K);
   if (form == 6) return igemm_launch_shared_tail<64, 128, CONV_BK>(al, bl, ep, M, N, K);
   if (form == 7) return igemm_launch_shared_tail<128, 128, CONV_BK>(al, bl, ep, M, N, K);
