@@ -33,7 +33,7 @@ class PyBuf:
         return Buf(self.ptr + 4 * int(k), self.n - int(k) if n is None else n, self.keep)
 
 
-Buf = PyBuf if _lib._lhpy is None else _lib._lhpy.Buf          # the same, without an entry in the garbage collector
+Buf = PyBuf if _lib._lhpy is None else _lib._lhpy.Buf          # the same, without an entry in the garbage collector where there is no owner
 
 
 _INTS_CACHE = {}

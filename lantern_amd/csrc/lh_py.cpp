@@ -163,14 +163,17 @@ PyObject* make_check(PyObject*, PyObject* args) {
   return (PyObject*)c;
 }
 
-// ---- Buf: a span of backend memory (address, number of 4-byte elements, an owner to keep alive); not followed by the collector ------
+// ---- Buf: a span of backend memory (address, number of 4-byte elements, an owner to keep alive).  The collector follows it only where
+// there is an owner (which may hold the Buf in turn): such a one is an OwnedBuf, the same for the caller.
 struct Buf { PyObject_HEAD PyObject *ptr, *n, *keep; };
 PyTypeObject BufType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+PyTypeObject OwnedBufType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 inline PyObject* as_int(PyObject* o) {
   if (PyLong_CheckExact(o)) { Py_INCREF(o); return o; }
   return PyNumber_Long(o);
 }
 PyObject* buf_of(PyTypeObject* type, PyObject* ptr, PyObject* n, PyObject* keep) {           // takes over ptr and n
+  if (type == &BufType && keep != Py_None) type = &OwnedBufType;
   Buf* b = ptr && n ? (Buf*)type->tp_alloc(type, 0) : nullptr;
   if (!b) { Py_XDECREF(ptr); Py_XDECREF(n); return nullptr; }
   Py_INCREF(keep);
@@ -204,6 +207,9 @@ void buf_dealloc(PyObject* self) {
   Py_XDECREF(b->ptr); Py_XDECREF(b->n); Py_XDECREF(b->keep);
   Py_TYPE(self)->tp_free(self);
 }
+void owned_buf_dealloc(PyObject* self) { PyObject_GC_UnTrack(self); buf_dealloc(self); }
+int buf_traverse(PyObject* self, visitproc visit, void* arg) { Buf* b = (Buf*)self; Py_VISIT(b->ptr); Py_VISIT(b->n); Py_VISIT(b->keep); return 0; }
+int buf_clear(PyObject* self) { Buf* b = (Buf*)self; Py_CLEAR(b->keep); return 0; }
 // offset(k, n=None): the same memory, starting k elements in
 PyObject* buf_offset(PyObject* self, PyObject* args, PyObject* kw) {
   static const char* names[] = {"k", "n", nullptr};
@@ -242,7 +248,11 @@ PyMODINIT_FUNC PyInit__lhpy(void) {
   BufType.tp_name = "lantern_amd.backend.Buf"; BufType.tp_basicsize = sizeof(Buf); BufType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_BASETYPE;
   BufType.tp_doc = "A span of backend memory: address, element count (4-byte elements) and an owner to keep alive.";
   BufType.tp_new = buf_new; BufType.tp_vectorcall = buf_vectorcall; BufType.tp_dealloc = buf_dealloc; BufType.tp_members = buf_members; BufType.tp_methods = buf_methods;
-  if (PyType_Ready(&CallType) < 0 || PyType_Ready(&CheckType) < 0 || PyType_Ready(&BufType) < 0) return nullptr;
+  BufType.tp_traverse = buf_traverse; BufType.tp_clear = buf_clear;           // (for classes derived from it, which the collector follows)
+  OwnedBufType.tp_name = BufType.tp_name; OwnedBufType.tp_basicsize = sizeof(Buf); OwnedBufType.tp_base = &BufType; OwnedBufType.tp_doc = BufType.tp_doc;
+  OwnedBufType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_BASETYPE | Py_TPFLAGS_HAVE_GC;
+  OwnedBufType.tp_dealloc = owned_buf_dealloc; OwnedBufType.tp_traverse = buf_traverse; OwnedBufType.tp_clear = buf_clear; OwnedBufType.tp_free = PyObject_GC_Del;
+  if (PyType_Ready(&CallType) < 0 || PyType_Ready(&CheckType) < 0 || PyType_Ready(&BufType) < 0 || PyType_Ready(&OwnedBufType) < 0) return nullptr;
   PyObject* m = PyModule_Create(&module);
   if (!m) return nullptr;
   Py_INCREF(&BufType);

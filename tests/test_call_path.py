@@ -1,7 +1,10 @@
 """The native call path (csrc/lh_py.cpp) against ctypes: the same values arrive for ordinary arguments, the same objects are refused."""
+import copy
 import ctypes as C
+import gc
 import shutil
 import subprocess
+import weakref
 
 import numpy as np
 import pytest
@@ -69,6 +72,30 @@ def test_handles(cls):
             cls(*bad)
     with pytest.raises(AttributeError):
         b.other = 1
+
+
+@pytest.mark.parametrize("cls", [B.PyBuf, B.Buf])
+def test_an_owner_that_holds_its_handle_is_collected(cls):
+    class Owner:
+        pass
+
+    class Derived(cls):
+        pass
+    for kind in (cls, Derived):
+        o = Owner()
+        o.buf = kind(4096, 10, o).offset(1)
+        assert isinstance(o.buf, (B.PyBuf, B.Buf)) and o.buf.keep is o
+        o.direct = kind(4096, 10, o)
+        gone = weakref.ref(o)
+        del o
+        gc.collect()
+        assert gone() is None
+    b = cls(4096, 10, keep=[1])
+    c = copy.copy(b)
+    assert (c.ptr, c.n, c.keep) == (4096, 10, [1]) and isinstance(b, cls) and isinstance(c, cls)
+    for _ in range(1000):
+        cls(1, 2, [b])
+    gc.collect()
 
 
 def test_tensors_still_take_attributes():
