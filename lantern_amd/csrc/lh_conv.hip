@@ -430,8 +430,8 @@ static bool launch_rounds(const AL& al, const BL& bl, const EP& ep, int M, int N
 // slices along the reduction and finished by whichever slice arrives last (igemm_launch_shared_tail).
 // 16-18: 64x64 tiles on blocks of two or four groups of wavefronts that share a tile's slabs (igemm_block): whole tiles on two and on
 // four, plan 13 on two; for launches of a few tiles per compute unit (beyond eight none of them was ever the fastest of a ResNet-50's
-// shapes) with at least four slabs a group.  Steps with them and without, one card in turn: ResNet-50 on 32x32 images 3.61 | 3.79 ms,
-// batch 21 at 161x161 6.27 | 6.39, batch 64 at 224x224 17.70 | 17.86, DeepSpeech 8.49 | 8.60.
+// shapes) with at least four slabs a group.  Steps with them and without, one card in turn: ResNet-50 on 32x32 images 3.61 | 3.79 ms
+// (batch 21 at 161x161 6.27 | 6.39, batch 64 at 224x224 17.70 | 17.86, DeepSpeech 8.49 | 8.60: 1 to 2 %, what runs differ by).
 constexpr int N_PLANS = 19;
 static inline bool deep_ok(int M, int N, int K, int groups) { return !g_deterministic && cdiv(K, CONV_BK) >= 4 * groups && cdiv(M, 64) * cdiv(N, 64) <= 8 * (int64_t)g_num_cu; }
 // LH_FORCE_M32 in the environment: products of at most 32 rows always take the 32-row tile (for tests of that tile; the

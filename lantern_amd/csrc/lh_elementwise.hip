@@ -469,8 +469,8 @@ __global__ void __launch_bounds__(TPB) k_col_finish(float* small, const float* _
 }
 // true: done.  Slices: a second launch costs 2.5 us, which a block of 16 wavefronts over up to 2048 rows is done in (2048x1000 6.6 us, 2
 // slices 6.6); beyond, a block per compute unit, four slices where there are columns enough (4096x50257 187 -> 172 us), 512 rows a block.
-// 8192x4096 23 us, 64x1000 4.0, 256x1000 4.1, 1000000x4 25 (a wavefront per column reading one element of a row at a time: 178, 4.2,
-// 5.0, 8306; with 8 chains a slice and slices of 64 rows in place of the pairs: 23, 3.7, 6.8, 133).
+// 8192x4096 23 us, 64x1000 3.4, 256x1000 3.4, 1000000x4 22 (a wavefront per column reading one element of a row at a time: 178, 4.2,
+// 5.0, 8306; with 8 chains a slice and slices of 64 rows in place of the pairs: 23, 3.5, 5.9, 133).
 static bool col_sums(float* small, const float* big, int rows, int cols, float sign) {
   const int gx = (int)cdiv(cols, 64);
   int slices = 1;

@@ -27,7 +27,7 @@
 // What bounds it is latency: of an Elman step's 2.4 us (B 32, H 800) the matrix instructions take 0.7, the rest is a word's way out
 // (a write-through store) and in (polls of 0.7 us a round), LDS and the activation.  Per step, one launch per step -> now, B 32,
 // H 800: Elman, both directions 5.1 -> 2.5 us, LSTM forward 9.4 -> 4.1, backward 14.8 -> 6.4 (3200 k, 100 blocks: 2.7 us of matrix
-// instructions).  DeepSpeech2 step 11.14 -> 7.9 ms, LSTM layer (T 185) 5.04 -> 2.77 ms, GRU 4.64 -> 2.5, hidden sizes that are no
+// instructions).  DeepSpeech2 step 11.24 -> 8.37 ms, LSTM layer (T 185) 5.04 -> 2.84, GRU 4.48 -> 2.47, hidden sizes that are no
 // multiple of 4 (which kept the per-step vector kernels or a cut product) 4 to 7 times as fast.  Measured and dropped: a slot per
 // step read through L2 once its first words are there (equal: bandwidth is not the bound), asking for one group first and the
 // rest behind it (equal to 4 % slower), waiting 0.2 to 0.9 us before the first poll (2 to 8 % slower), sc1 alone (equal).
