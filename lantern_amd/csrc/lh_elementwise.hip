@@ -481,6 +481,7 @@ static bool col_sums(float* small, const float* big, int rows, int cols, float s
     if (slices > 256) slices = 256;
   }
   const int per = (int)cdiv(rows, slices);
+  if ((int64_t)rows + per > 0x7fff0000) return false;     // (row numbers past the last of a slice stay within 32 bits)
   slices = (int)cdiv(rows, per);
   bool side = false;
   const size_t bytes = slices > 1 ? (size_t)slices * cols * sizeof(float) : 0;
