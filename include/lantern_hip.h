@@ -181,7 +181,7 @@ void lh_prof_collect(double* h_ms, int64_t* h_calls, int ncat);
  *     nor, under a join, the batch norm's.  Producing those afterwards means running the convolution again: when they are read, when
  *     their operands are overwritten while they could still be read (buffers that are used again instead of released by lh_rewind),
  *     or by an lh_flush_deferred in front of the lh_rewind.  A filter to which that has happened once has its calls run as issued
- *     from then on, until it is released.
+ *     from then on, until it is released or lh_set_fusion is called.
  *   - the copies of a filter in the layouts the convolution kernels read (tap-major for the forward pass, transposed per
  *     stride class for the input gradient) are kept, in device memory of their own outside the arena (at most 1 GiB together),
  *     while nothing writes the filter: any call of this header that writes into the filter's range ends them, and so does a

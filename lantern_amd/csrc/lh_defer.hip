@@ -652,6 +652,7 @@ void lh_set_fusion(int on) {
   lazy::Scope s_;
   lazy::flush_all();
   lazy::layouts_all_stale();
+  lazy::filters_released(nullptr);
   lazy::refresh_busy();
   lazy::g_enabled = on != 0;
 }
