@@ -51,6 +51,8 @@ static std::vector<ZeroBlock> g_zero;          // ascending addresses: the arena
 
 enum { V_MASK = 0, V_BN_OUT = 1, V_CONV = 2, V_BN_INFER = 3 };
 struct ConvArgs { const float* x; const float* w; const float* bias; float* y; int N, C, H, W, K, R, S, sH, sW, pH, pW, P, Q; };
+// Memory the arena gives up when its top falls to `from`.  (Operands may lie outside the arena: those stay, whatever their address.)
+static inline bool released(const void* p, const char* from) { return (const char*)p >= from && (const char*)p < arena_end(); }
 struct Unwritten {
   int kind; char* dst; size_t bytes;
   const float* src; const float* y; int64_t n;                                           // V_MASK: dst = y > 0 ? src : 0
@@ -602,22 +604,23 @@ void reset() { g_p = Parked(); g_zero.clear(); g_unwritten.clear(); g_records.cl
 static void produce_from_released(const char* from) {
   for (size_t i = 0; i < g_unwritten.size();) {
     const Unwritten& v = g_unwritten[i];
-    const bool gone = v.kind == V_CONV ? ((const char*)v.conv.x >= from || (const char*)v.conv.w >= from || (const char*)v.conv.bias >= from)
-                                       : v.kind == V_BN_INFER && ((const char*)v.x >= from || (const char*)v.gamma >= from || (const char*)v.beta >= from || (const char*)v.sm >= from || (const char*)v.si >= from);
-    if (gone && v.dst < from) { const Unwritten copy = v; g_unwritten.erase(g_unwritten.begin() + i); produce(copy); i = 0; } else i++;
+    const bool gone = v.kind == V_CONV ? released(v.conv.x, from) || released(v.conv.w, from) || released(v.conv.bias, from)
+                                       : v.kind == V_BN_INFER && (released(v.x, from) || released(v.gamma, from) || released(v.beta, from) || released(v.sm, from) || released(v.si, from));
+    if (gone && !released(v.dst, from)) { const Unwritten copy = v; g_unwritten.erase(g_unwritten.begin() + i); produce(copy); i = 0; } else i++;
   }
 }
-void filters_released(const char* from) { if (!g_wanted.empty()) g_wanted.erase(g_wanted.lower_bound(from), g_wanted.end()); }
+void filters_released(const char* from) { if (!g_wanted.empty()) g_wanted.erase(g_wanted.lower_bound(from), g_wanted.lower_bound(arena_end())); }
 void arena_released(char* from) {
   if (!g_unwritten.empty()) produce_from_released(from);
   filters_released(from);
   if (!g_layouts.empty()) layouts_released(from);
   while (!g_zero.empty() && g_zero.back().p >= from) g_zero.pop_back();
   for (size_t i = 0; i < g_unwritten.size();) {
-    if (g_unwritten[i].dst >= from) g_unwritten.erase(g_unwritten.begin() + i); else i++;
+    if (released(g_unwritten[i].dst, from)) g_unwritten.erase(g_unwritten.begin() + i); else i++;
   }
   for (size_t i = 0; i < g_records.size();) {
-    if ((const char*)g_records[i].y >= from) g_records.erase(g_records.begin() + i); else i++;
+    const FwdRecord& r = g_records[i];
+    if (released(r.y, from) || released(r.x, from) || released(r.bias, from)) g_records.erase(g_records.begin() + i); else i++;
   }
   refresh_busy();
 }
@@ -627,15 +630,15 @@ void on_rewind(char* new_top) {
   // would have to produce every unwritten batch-norm output that depends on the parameters it changes, for nobody to read.
   bool keep = g_p.kind == P_UPDATE;
   if (keep) for (size_t i = 0; i < g_p.ux.size(); i++) {
-    if ((char*)g_p.ux[i] >= new_top || (char*)g_p.ud[i] >= new_top || (g_p.uv[i] && (char*)g_p.uv[i] >= new_top)) { keep = false; break; }
+    if (released(g_p.ux[i], new_top) || released(g_p.ud[i], new_top) || released(g_p.uv[i], new_top)) { keep = false; break; }
   }
   if (!keep) flush_parked();
   arena_released(new_top);
   // a result kept below the new top whose recipe reads released memory is produced now
   for (size_t i = 0; i < g_unwritten.size();) {
     const Unwritten& v = g_unwritten[i];
-    const bool dangling = v.kind == V_MASK ? ((const char*)v.src >= new_top || (const char*)v.y >= new_top)
-                                           : v.kind == V_BN_OUT && ((const char*)v.x >= new_top || (const char*)v.sm >= new_top || (const char*)v.si >= new_top);
+    const bool dangling = v.kind == V_MASK ? released(v.src, new_top) || released(v.y, new_top)
+                                           : v.kind == V_BN_OUT && (released(v.x, new_top) || released(v.sm, new_top) || released(v.si, new_top));
     if (dangling) { const Unwritten copy = v; g_unwritten.erase(g_unwritten.begin() + i); produce(copy); i = 0; } else i++;
   }
   refresh_busy();
@@ -652,7 +655,7 @@ void lh_set_fusion(int on) {
   lazy::Scope s_;
   lazy::flush_all();
   lazy::layouts_all_stale();
-  lazy::filters_released(nullptr);
+  lazy::g_wanted.clear();
   lazy::refresh_busy();
   lazy::g_enabled = on != 0;
 }

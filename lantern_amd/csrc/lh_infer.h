@@ -13,6 +13,7 @@ __attribute__((weak)) void bn_infer_now(const float* x, const float* gamma, cons
                                         int relu, int N, int C, int HW);
 namespace lazy {
 bool park_bn_infer(const float* x, const float* gamma, const float* beta, const float* mean, const float* var, float* y, int N, int C, int HW, float eps);
-void filters_released(const char* from);       // filters above `from` are gone: what is remembered of their chains goes too
+void filters_released(const char* from);       // the arena above `from` is released: what is remembered of the chains of filters there goes too
 }
+const char* arena_end();
 }  // namespace lh

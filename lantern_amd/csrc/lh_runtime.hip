@@ -143,6 +143,7 @@ static void zero_async(void* p, size_t bytes) {  // bytes is a multiple of 256
   hipLaunchKernelGGL(k_zero16, dim3(grid), dim3(256), 0, g_stream, (uint4*)p, n16);
 }
 size_t arena_room() { return g_arena.bytes - g_arena.top; }
+const char* arena_end() { return g_heap + g_arena.bytes; }
 void zero_bytes_async(void* p, size_t bytes) { ProfScope prof_(CAT_FILL); zero_async(p, bytes); }
 }  // namespace lh
 using namespace lh;

@@ -157,6 +157,42 @@ def test_the_form_is_measured_for_any_channel_count(on_hip, case):
 
 
 @pytest.mark.gpu
+def test_outputs_outside_the_arena_outlast_a_rewind(on_hip):
+    """A rewind releases arena memory: outputs of a chain in memory of the caller's own are there behind it, stored or not."""
+    import torch
+    be, lib = on_hip, on_hip.lib
+    rng = np.random.RandomState(4)
+    N, C, H, K = 2, 16, 8, 32
+    n = N * K * H * H
+    up = lambda a: be.fromHost(np.ascontiguousarray(a.astype(np.float32)))      # noqa: E731
+    x, w = up(rng.standard_normal((N, C, H, H))), up(rng.standard_normal((K, C, 3, 3)))
+    g, b, m, v, sc = up(rng.standard_normal(K)), up(rng.standard_normal(K)), up(rng.standard_normal(K)), up(rng.uniform(0.5, 1, K)), up(rng.standard_normal(n))
+    dims = B._ints((n,))
+    results = []
+    try:
+        be.setDeterministic(True)
+        for fusion in (0, 1):
+            lib.lh_set_fusion(fusion)
+            own = [torch.full((n,), 7.0, device="cuda") for _ in range(3)]
+            torch.cuda.synchronize()
+            y, t, o = (B.Buf(a.data_ptr(), n, a) for a in own)
+            mark = be.getMallocAddr()
+            be.mallocArray(1 << 20)
+            lib.lh_conv2d_fwd(x.ptr, w.ptr, 0, y.ptr, N, C, H, H, K, 3, 3, 1, 1, 1, 1)
+            lib.lh_bn_infer(y.ptr, g.ptr, b.ptr, m.ptr, v.ptr, t.ptr, N, K, H * H, 1e-5)
+            lib.lh_bcast_op(B.ADD, t.ptr, dims, sc.ptr, dims, o.ptr, dims, 1)
+            lib.lh_unary(B.RELU, o.ptr, o.ptr, n, 0.0, 0.0)
+            _lib.check()
+            be.resetMallocAddr(mark)
+            results.append([be.toHost(a, n) for a in (y, t, o)])
+    finally:
+        lib.lh_set_fusion(1)
+        be.setDeterministic(False)
+    for a, c in zip(*results):
+        np.testing.assert_array_equal(a, c)
+
+
+@pytest.mark.gpu
 def test_infinities_and_nan_pass_as_through_the_parts(on_hip):
     be, lib = on_hip, on_hip.lib
     mark = be.getMallocAddr()
