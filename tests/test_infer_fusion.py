@@ -159,7 +159,7 @@ def test_the_form_is_measured_for_any_channel_count(on_hip, case):
 @pytest.mark.gpu
 def test_outputs_outside_the_arena_outlast_a_rewind(on_hip):
     """A rewind releases arena memory: outputs of a chain in memory of the caller's own are there behind it, stored or not."""
-    import torch
+    import ctypes
     be, lib = on_hip, on_hip.lib
     rng = np.random.RandomState(4)
     N, C, H, K = 2, 16, 8, 32
@@ -168,14 +168,17 @@ def test_outputs_outside_the_arena_outlast_a_rewind(on_hip):
     x, w = up(rng.standard_normal((N, C, H, H))), up(rng.standard_normal((K, C, 3, 3)))
     g, b, m, v, sc = up(rng.standard_normal(K)), up(rng.standard_normal(K)), up(rng.standard_normal(K)), up(rng.uniform(0.5, 1, K)), up(rng.standard_normal(n))
     dims = B._ints((n,))
+    own = [ctypes.c_void_p() for _ in range(3)]
+    for a in own:
+        assert lib["hipMalloc"](ctypes.byref(a), ctypes.c_size_t(4 * n)) == 0          # (of the runtime the library is linked with)
     results = []
     try:
         be.setDeterministic(True)
         for fusion in (0, 1):
             lib.lh_set_fusion(fusion)
-            own = [torch.full((n,), 7.0, device="cuda") for _ in range(3)]
-            torch.cuda.synchronize()
-            y, t, o = (B.Buf(a.data_ptr(), n, a) for a in own)
+            y, t, o = (B.Buf(own[i].value, n) for i in range(3))
+            for a in (y, t, o):
+                be.fillInPlace(a, n, 7.0)
             mark = be.getMallocAddr()
             be.mallocArray(1 << 20)
             lib.lh_conv2d_fwd(x.ptr, w.ptr, 0, y.ptr, N, C, H, H, K, 3, 3, 1, 1, 1, 1)
@@ -188,6 +191,9 @@ def test_outputs_outside_the_arena_outlast_a_rewind(on_hip):
     finally:
         lib.lh_set_fusion(1)
         be.setDeterministic(False)
+        be.sync()
+        for a in own:
+            lib["hipFree"](a)
     for a, c in zip(*results):
         np.testing.assert_array_equal(a, c)
 
